@@ -13,7 +13,8 @@
 //   out[d, c, o] = sum_{e -> d} sum_p R[e,c,p] sum_{(a,b) in p -> o} CG x[src_e,c,a] Y_e[b]
 //
 // Work per edge: the MLP's second layer is a GEMM [edges x 64] x [64 x 34C]
-// (557 kflop per edge at C = 128).  One kernel per pass runs it on MFMA and
+// (557 kflop per edge at C = 128).  One kernel per pass runs it on the bf16 matrix
+// cores (each fp32 operand as three bf16 parts, six products: common.h) and
 // consumes each tile of per-edge weights R straight from the accumulators in
 // the channel-wise CG product on the VALU (611 products with a coefficient,
 // 256 bilinear products and 156 path weightings per edge and channel), so R
@@ -401,16 +402,22 @@ __global__ void mace_reverse_edges_kernel(const int64_t* __restrict__ row_ptr,
 // [E][64] (the backward also s[E][64], below).
 //
 // A workgroup owns one quad of 4 channels c0..c0+3 and keeps that quad's slice
-// of W2 in LDS as sW[g][4 ch + j][k] = W2[k][(4g + j) C + c0 + ch] (paths in 9
-// groups of 4, the last two slots zero; rows of 68 floats).  Each of its 4
-// waves walks its own range of positions (ranges end at destination
-// boundaries) in tiles of 16 edges.  Per tile, v_mfma_f32_16x16x4f32 gives
+// of W2 in LDS, split into bf16 parts, as MFMA operand fragments (paths in 9 groups
+// of 4, the last two slots zero).  Each of its waves walks its own range of positions
+// (ranges end at destination boundaries) in tiles of 16 edges.  Per tile,
+// v_mfma_f32_16x16x32_bf16 gives
 //   D[4 ch + j][e] = sum_k W2[k][(4g + j) C + c0 + ch] h[e][k]  = R[e, c0 + ch, 4g + j]
-// (A = the W2 rows from LDS, B = h of the tile, K = 64 in 16 steps, 9 groups:
-// 144 MFMAs), and by the accumulator layout lane l = 16 ch + e holds the 34
-// weights of its own (edge e, channel c0 + ch) pair.  The lane then forms the
-// message of that pair, sum_p R_p T_p(x[src, c], Y(u)), on the VALU.
-// R never leaves the registers.
+// (A = the W2 fragments from LDS, B = h of the tile, K = 64 in 2 steps of 6 products,
+// 9 groups: 108 MFMAs of 16 cycles, against 144 of 32 with fp32 MFMAs), and by the
+// accumulator layout lane l = 16 ch + e holds the 34 weights of its own (edge e,
+// channel c0 + ch) pair.  The lane then forms the message of that pair,
+// sum_p R_p T_p(x[src, c], Y(u)), on the VALU.  R never leaves the registers.
+//
+// Bound: VALU + MFMA issue of the SIMD, which overlap little (a probe: 8 FMAs between
+// 16-cycle MFMAs add their whole time with 4 waves per SIMD).  N = 50,000, C = 128,
+// 1.5 M edges: forward kernel 10.5 -> 7.4 ms, backward 17.9 -> 12.6 ms against the fp32
+// MFMA form, the layer's pass 29.0 -> 20.9 ms, its error against 64 bits unchanged
+// (9.8e-7; it comes from the radial basis).
 //
 // Each destination's messages are summed in ascending edge order by one lane
 // after another along the tile (lane e adds lane e - 1's running sum when both
@@ -419,48 +426,70 @@ __global__ void mace_reverse_edges_kernel(const int64_t* __restrict__ row_ptr,
 // sequence of additions whatever the tiling, the order of the destinations or
 // the launch shape; each output row is written once, with no atomics.
 // ---------------------------------------------------------------------------
-constexpr int kMaceFwdWaves = 8;                     // waves (position ranges) per workgroup
-constexpr int kMaceBwdWaves = 4;
+constexpr int kMaceFwdWaves = 16;                    // waves (position ranges) per workgroup
+constexpr int kMaceBwdWaves = 12;
 constexpr int kPG = 9;                               // groups of 4 paths (36 slots)
-constexpr int kW2Row = kHidden + 4;                  // LDS row of sW, in floats
-constexpr int kW2Floats = kPG * 16 * kW2Row;         // 39,168 bytes per channel quad
+constexpr int kHSteps = kHidden / 32;                // K = 32 steps of the hidden layer
+constexpr int kHRow = 3 * kHidden / 8;               // h of a position: 24 v4u, [part][k / 8]
+constexpr int kW2Frags = kPG * kHSteps * 3;          // 1 KB operand fragments per channel quad
 constexpr int kMaceMaxWorkers = 8192;                // position ranges (wstart entries - 1)
 
-// sW for the channel quad c0..c0+3 (zeros past path 33 and past channel C - 1)
+// The quad's W2 slice as MFMA operand fragments, sW[(g * 2 + s) * 3 + part][lane]: row
+// lane % 16 = 4 ch + j of group g (path 4g + j of channel c0 + ch), hidden units
+// 32 s + 8 (lane / 16) .. + 7 (zeros past path 33 and past channel C - 1).
 __device__ __forceinline__ void mace_fill_w2(const float* __restrict__ w2, int C, int c0,
-                                             float* sW) {
-    for (int i = threadIdx.x; i < kHidden * 36 * 4; i += blockDim.x) {
-        const int ch = i & 3, p = (i >> 2) % 36, k = i / 144;
-        const int c = c0 + ch;
-        float v = 0.0f;
-        if (p < kNumPaths && c < C) v = w2[(int64_t)k * kNumPaths * C + p * C + c];
-        sW[((p >> 2) * 16 + 4 * ch + (p & 3)) * kW2Row + k] = v;
+                                             v4u* sW) {
+    for (int i = threadIdx.x; i < kPG * kHSteps * 64; i += blockDim.x) {
+        const int lane = i & 63, s = (i >> 6) % kHSteps, g = (i >> 6) / kHSteps;
+        const int c = c0 + ((lane & 15) >> 2), p = 4 * g + (lane & 3);
+        const int k0 = 32 * s + 8 * (lane >> 4);
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            v[j] = p < kNumPaths && c < C ? w2[((int64_t)(k0 + j) * kNumPaths + p) * C + c] : 0.0f;
+        const Bf3 b = bf16_split8(v);
+        v4u* f = sW + (g * kHSteps + s) * 3 * 64 + lane;
+        f[0] = b.h;
+        f[64] = b.m;
+        f[128] = b.l;
     }
 }
 
-// The 34 weights of the lane's pair: sA = sW + (lane % 16) row + 4 (lane / 16),
-// hb[j] = h[e][16 j + 4 (lane / 16) .. + 3] (k-step s of block j is
-// k = 16 j + 4 (lane / 16) + s for both operands).
-__device__ __forceinline__ void mace_tile_weights(const float* sA, const float4* hb, float* rr) {
+// The 34 weights of the lane's pair: sA = sW + lane, hb[part * 2 + s] = the part of
+// h[e][32 s + 8 (lane / 16) .. + 7].  The small products of both K steps go first, while
+// the accumulator is small.
+__device__ __forceinline__ void mace_tile_weights(const v4u* sA, const v4u* hb, float* rr) {
     // the W2 operands are the same for every tile: read them from LDS per tile (an
-    // opaque base keeps the compiler from hoisting all 36 reads, 144 registers, out
-    // of the tile loop)
+    // opaque base keeps the compiler from hoisting the reads out of the tile loop)
     int base = 0;
     asm volatile("" : "+v"(base));
     sA += base;
-    v4f acc[kPG];
+    static_for<kPG>([&](auto gg) {
+        constexpr int g = decltype(gg)::value;
+        v4u a[3 * kHSteps];
 #pragma unroll
-    for (int g = 0; g < kPG; ++g) acc[g] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < kHSteps; ++s)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+            for (int q = 0; q < 3; ++q) a[q * kHSteps + s] = sA[((g * kHSteps + s) * 3 + q) * 64];
+        v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int g = 0; g < kPG; ++g) {
-            const float4 a = *reinterpret_cast<const float4*>(sA + g * 16 * kW2Row + 16 * j);
-            acc[g] = mfma4(a, hb[j], acc[g]);
+        for (int s = 0; s < kHSteps; ++s) {
+            acc = mfma_bf16(a[2 * kHSteps + s], hb[s], acc);
+            acc = mfma_bf16(a[s], hb[2 * kHSteps + s], acc);
+            acc = mfma_bf16(a[kHSteps + s], hb[kHSteps + s], acc);
         }
-    }
 #pragma unroll
-    for (int p = 0; p < kNumPaths; ++p) rr[p] = acc[p >> 2][p & 3];
+        for (int s = 0; s < kHSteps; ++s) {
+            acc = mfma_bf16(a[kHSteps + s], hb[s], acc);
+            acc = mfma_bf16(a[s], hb[kHSteps + s], acc);
+        }
+#pragma unroll
+        for (int s = 0; s < kHSteps; ++s) acc = mfma_bf16(a[s], hb[s], acc);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (4 * g + j < kNumPaths) rr[4 * g + j] = acc[j];
+        __builtin_amdgcn_sched_barrier(0);  // one group's fragments at a time
+    });
 }
 
 // Lane reads within the 16-lane row.  Call them where every lane runs (a lane that
@@ -475,7 +504,7 @@ __device__ __forceinline__ int dpp_next_i(int v) {  // lane e + 1 of the 16-lane
 
 // One tile's per-position operands (pos clamped into the range by the caller).
 struct MaceTileIn {
-    float4 hb[4];
+    v4u hb[3 * kHSteps];
     float4 u;  // unit vector, length
     int s, d;
 };
@@ -483,11 +512,11 @@ struct MaceTileIn {
 __device__ __forceinline__ void mace_load_tile(const float4* __restrict__ u4,
                                                const int* __restrict__ srcp,
                                                const int* __restrict__ dstp,
-                                               const float* __restrict__ h, int64_t pos, int kk,
+                                               const v4u* __restrict__ h, int64_t pos, int kk,
                                                MaceTileIn& t) {
-    const float4* hr = reinterpret_cast<const float4*>(h + pos * kHidden + 4 * kk);
+    const v4u* hr = h + pos * kHRow + kk;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) t.hb[j] = hr[4 * j];
+    for (int j = 0; j < 3 * kHSteps; ++j) t.hb[j] = hr[4 * j];
     t.u = u4[pos];
     t.s = srcp[pos];
     t.d = dstp[pos];
@@ -554,11 +583,11 @@ __device__ __forceinline__ MaceWg mace_wg(int n_quads, int ranges_per_xcd) {
 // destination with an edge (out of the others is zeroed by the caller).
 __global__ __launch_bounds__(64 * kMaceFwdWaves) __attribute__((amdgpu_waves_per_eu(4))) void
 mace_fused_forward_kernel(const float4* __restrict__ u4, const int* __restrict__ srcp,
-                          const int* __restrict__ dstp, const float* __restrict__ h,
+                          const int* __restrict__ dstp, const v4u* __restrict__ h,
                           const float* __restrict__ w2, const float* __restrict__ x,
                           const int64_t* __restrict__ wstart, float* __restrict__ out, int C,
                           int n_quads, int ranges_per_xcd) {
-    __shared__ __attribute__((aligned(16))) float sW[kW2Floats];
+    __shared__ v4u sW[kW2Frags * 64];
     __shared__ __attribute__((aligned(16))) float sTAll[kMaceFwdWaves * 4 * kTRow];
     const MaceWg wg = mace_wg<kMaceFwdWaves>(n_quads, ranges_per_xcd);
     const int lane = threadIdx.x & 63, e16 = lane & 15, kk = lane >> 4;
@@ -570,22 +599,23 @@ mace_fused_forward_kernel(const float4* __restrict__ u4, const int* __restrict__
     const int c = c0 + kk;
     const bool cok = c < C;
     const int cc = cok ? c : C - 1;
-    const float* sA = sW + (lane & 15) * kW2Row + 4 * kk;
+    const v4u* sA = sW + lane;
     int carry_d = -1;
     float acc = 0.0f;
     MaceTileIn cur;
     if (p0 < p1) mace_load_tile(u4, srcp, dstp, h, min(p0 + e16, p1 - 1), kk, cur);
     for (int64_t t0 = p0; t0 < p1; t0 += 16) {
         const bool valid = t0 + e16 < p1;
-        // source row of the pair (issued first: the MFMAs below hide its latency)
-        float xs[16];
-        load_row16(x + ((int64_t)cur.s * C + cc) * 16, xs);
         if (!valid) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) cur.hb[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int j = 0; j < 3 * kHSteps; ++j) cur.hb[j] = v4u{0, 0, 0, 0};
         }
         float rr[kNumPaths];
         mace_tile_weights(sA, cur.hb, rr);
+        // source row of the pair (after the weights: before them its 16 registers spill;
+        // the other waves of the SIMD cover its latency)
+        float xs[16];
+        load_row16(x + ((int64_t)cur.s * C + cc) * 16, xs);
         float Y[16];
         sh_forward<3>(cur.u.x, cur.u.y, cur.u.z, Y);
         float m[16];
@@ -602,31 +632,72 @@ mace_fused_forward_kernel(const float4* __restrict__ u4, const int* __restrict__
     if (carry_d >= 0 && cok) out[((int64_t)carry_d * C + c) * 16 + e16] = acc;
 }
 
+// Place of path p in the order in which mace_grad_y completes the paths (l1, l_out, l2).
+constexpr int grad_slot(int p) {
+    auto key = [](int i) { return (kPathL[i][0] * 4 + kPathL[i][2]) * 4 + kPathL[i][1]; };
+    int n = 0;
+    for (int i = 0; i < kNumPaths; ++i) n += key(i) < key(p) ? 1 : 0;
+    return n;
+}
+struct GradPaths {
+    int path[kNumPaths];
+    constexpr GradPaths() : path{} {
+        for (int p = 0; p < kNumPaths; ++p) path[grad_slot(p)] = p;
+    }
+};
+__constant__ constexpr GradPaths kGradPaths{};
+constexpr int kPOct = (kNumPaths + 7) / 8;           // octets of those places
+constexpr int kW2tFrags = kPOct * 4 * 3;
+
+// The quad's W2 slice as operand fragments of the transpose GEMM, sV[(q * 4 + j) * 3 +
+// part][lane]: row k = 16 j + lane % 16, places 8q .. 8q + 7 of channel c0 + lane / 16.
+__device__ __forceinline__ void mace_fill_w2t(const float* __restrict__ w2, int C, int c0,
+                                              v4u* sV) {
+    for (int i = threadIdx.x; i < kPOct * 4 * 64; i += blockDim.x) {
+        const int lane = i & 63, j = (i >> 6) & 3, q = i >> 8;
+        const int c = c0 + (lane >> 4), k = 16 * j + (lane & 15);
+        float v[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const int i = 8 * q + t;
+            v[t] = i < kNumPaths && c < C
+                       ? w2[((int64_t)k * kNumPaths + kGradPaths.path[i]) * C + c] : 0.0f;
+        }
+        const Bf3 b = bf16_split8(v);
+        v4u* f = sV + (q * 4 + j) * 3 * 64 + lane;
+        f[0] = b.h;
+        f[64] = b.m;
+        f[128] = b.l;
+    }
+}
+
 // Backward: per pair, gR_p = sum_o g[d, c, o] T_p[o] feeds the MLP's transpose GEMM
-//   D[k][e] += sum_{ch} W2[k][p C + c0 + ch] gR[e, c0 + ch, p]   (K = the quad's 4
-// channels, one MFMA per path and 16-row block of k: A = W2 from LDS, B = the lane's
-// own gR_p), and gY[b] = sum c x[a] R_p g[o] is summed over the quad's channels.
+//   D[k][e] += sum_{ch, p} W2[k][p C + c0 + ch] gR[e, c0 + ch, p]   (K step q = the
+// paths of places 8q .. 8q + 7, of the quad's 4 channels, by 16-row blocks of k: A = W2 from LDS, B = the
+// lane's own 8 gR_p), and gY[b] = sum c x[a] R_p g[o] is summed over the quad's channels.
 // The quad's share of the edge's position gradient,
 //   g_v = g_r u + (g_u - u (u . g_u)) / r,  g_r = sum_k D[k][e] s[e][k],
 //   g_u = SH backward of gY at u,
 // with s[e][k] = silu'(z_k) sum_b W1[b][k] dB_b/dr, goes to gv_part[quad][position].
 __global__ __launch_bounds__(64 * kMaceBwdWaves) __attribute__((amdgpu_waves_per_eu(3))) void mace_fused_backward_kernel(
     const float4* __restrict__ u4, const int* __restrict__ srcp, const int* __restrict__ dstp,
-    const float* __restrict__ h, const float* __restrict__ sg, const float* __restrict__ w2,
+    const v4u* __restrict__ h, const float* __restrict__ sg, const float* __restrict__ w2,
     const float* __restrict__ x, const float* __restrict__ gout,
     const int64_t* __restrict__ wstart, float* __restrict__ gv_part, int64_t n_pos, int C,
     int n_quads, int ranges_per_xcd) {
-    __shared__ __attribute__((aligned(16))) float sW[kW2Floats];
+    __shared__ v4u sW[kW2Frags * 64];
+    __shared__ v4u sV[kW2tFrags * 64];
     const MaceWg wg = mace_wg<kMaceBwdWaves>(n_quads, ranges_per_xcd);
     const int lane = threadIdx.x & 63, e16 = lane & 15, kk = lane >> 4;
     const int c0 = wg.quad * 4;
     mace_fill_w2(w2, C, c0, sW);
+    mace_fill_w2t(w2, C, c0, sV);
     __syncthreads();
     const int64_t p0 = wstart[wg.wave_range], p1 = wstart[wg.wave_range + 1];
     const int c = c0 + kk;
     const bool cok = c < C;
     const int cc = cok ? c : C - 1;
-    const float* sA = sW + (lane & 15) * kW2Row + 4 * kk;
+    const v4u* sA = sW + lane;
     float* gvq = gv_part + (int64_t)wg.quad * n_pos * 3;
     MaceTileIn cur;
     if (p0 < p1) mace_load_tile(u4, srcp, dstp, h, min(p0 + e16, p1 - 1), kk, cur);
@@ -639,7 +710,7 @@ __global__ __launch_bounds__(64 * kMaceBwdWaves) __attribute__((amdgpu_waves_per
         load_row16(gout + ((int64_t)cur.d * C + cc) * 16, g);
         if (!valid) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) cur.hb[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int j = 0; j < 3 * kHSteps; ++j) cur.hb[j] = v4u{0, 0, 0, 0};
         }
         float rr[kNumPaths];
         mace_tile_weights(sA, cur.hb, rr);
@@ -649,20 +720,32 @@ __global__ __launch_bounds__(64 * kMaceBwdWaves) __attribute__((amdgpu_waves_per
         }
         float Y[16];
         sh_forward<3>(cur.u.x, cur.u.y, cur.u.z, Y);
-        // gY of the pair, and gR_p = g . T_p per path straight into the transpose GEMM
+        // gY of the pair, and gR_p = g . T_p per path, every eight into the transpose GEMM
         v4f gh[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) gh[j] = v4f{0.f, 0.f, 0.f, 0.f};
-        float gy[16];
+        float gy[16], gR[8];
         // (W2 read per tile through an opaque base, as in mace_tile_weights)
         int wbase = 0;
         asm volatile("" : "+v"(wbase));
-        const float* sWt = sW + wbase;
+        const v4u* sVt = sV + lane + wbase;
         mace_grad_y(xs, g, Y, rr, gy, [&](auto pp, float gr) {
-            constexpr int p = decltype(pp)::value;
-            const float* a = sWt + ((p >> 2) * 16 + 4 * kk + (p & 3)) * kW2Row + e16;
+            constexpr int i = grad_slot(decltype(pp)::value), q = i / 8;
+            gR[i % 8] = gr;
+            if constexpr (i % 8 == 7 || i == kNumPaths - 1) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) gh[j] = mfma1(a[16 * j], gr, gh[j]);
+                for (int z = i % 8 + 1; z < 8; ++z) gR[z] = 0.0f;
+                // (barriers: hoisted into the products, the fragments' reads spill)
+                __builtin_amdgcn_sched_barrier(0);
+                const Bf3 b = bf16_split8_finite(gR);
+                static_for<4>([&](auto jj) {
+                    constexpr int j = decltype(jj)::value;
+                    const v4u* f = sVt + (q * 4 + j) * 3 * 64;
+                    const Bf3 a{f[0], f[64], f[128]};
+                    mfma_bf16x6(a, b, gh[j], gh[j]);
+                    if constexpr (j % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+                });
+            }
         });
         // the next tile's operands and this tile's s, in flight during the reductions
         MaceTileIn nxt;
@@ -764,7 +847,7 @@ __global__ __launch_bounds__(256) void mace_prep_kernel(
     const int64_t* __restrict__ dst, const int64_t* __restrict__ perm,
     const float* __restrict__ w1, const float* __restrict__ b1, float rc, int64_t n_edges,
     float4* __restrict__ u4, int* __restrict__ srcp, int* __restrict__ dstp,
-    float* __restrict__ h, float* __restrict__ sg) {
+    v4u* __restrict__ h, float* __restrict__ sg) {
     __shared__ float sW[kNBasis * kHidden + kHidden];
     for (int i = threadIdx.x; i < kNBasis * kHidden + kHidden; i += blockDim.x)
         sW[i] = i < kNBasis * kHidden ? w1[i] : b1[i - kNBasis * kHidden];
@@ -824,8 +907,14 @@ __global__ __launch_bounds__(256) void mace_prep_kernel(
             sd[t] = sgm * (1.0f + acc * (1.0f - sgm)) * qq;
         }
     }
+    // h in three bf16 parts, [part][k] (hidden units 4q .. 4q + 3 of each part here)
+    const float z8[8] = {z[0], z[1], z[2], z[3], 0.f, 0.f, 0.f, 0.f};
+    const Bf3 zs = bf16_split8(z8);
     if (valid) {
-        reinterpret_cast<float4*>(h + p * kHidden)[q] = make_float4(z[0], z[1], z[2], z[3]);
+        uint2* hr = reinterpret_cast<uint2*>(h + p * kHRow) + q;
+        hr[0] = make_uint2(zs.h[0], zs.h[1]);
+        hr[kHidden / 4] = make_uint2(zs.m[0], zs.m[1]);
+        hr[kHidden / 2] = make_uint2(zs.l[0], zs.l[1]);
         if (sg) reinterpret_cast<float4*>(sg + p * kHidden)[q] = make_float4(sd[0], sd[1], sd[2], sd[3]);
     }
 }
@@ -873,7 +962,8 @@ struct MaceWs {
     int64_t *deg, *pos0, *perm, *wstart;
     float4* u4;
     int *srcp, *dstp;
-    float *h, *sg, *gv_part, *gv;
+    v4u* h;
+    float *sg, *gv_part, *gv;
     size_t bytes;
 };
 
@@ -898,7 +988,7 @@ static MaceWs mace_ws(void* base, int64_t N, int64_t E, int C, bool backward) {
     w.u4 = static_cast<float4*>(take(sizeof(float4) * e));
     w.srcp = static_cast<int*>(take(sizeof(int) * e));
     w.dstp = static_cast<int*>(take(sizeof(int) * e));
-    w.h = static_cast<float*>(take(sizeof(float) * kHidden * e));
+    w.h = static_cast<v4u*>(take(sizeof(v4u) * kHRow * e));
     if (backward) {
         w.sg = static_cast<float*>(take(sizeof(float) * kHidden * e));
         w.gv_part = static_cast<float*>(take(sizeof(float) * 3 * e * (size_t)mace_quads(C)));
@@ -934,9 +1024,12 @@ static int mace_cu_count() {
     return n;
 }
 
-// Launch shape of a fused kernel: every quad of a position range on one XCD, as
-// many ranges per XCD as fill one round of resident workgroups (occupancy from the
-// runtime for this kernel), so no second, partly idle round follows.
+// Launch shape of a fused kernel: every quad of a position range on one XCD.  The
+// workgroups of an XCD, ranges x quads, run in rounds of its resident ones (occupancy
+// from the runtime for this kernel); a range is a 1 / ranges share of the work, so the
+// time goes as rounds / ranges.  The ranges are the fewest that bring it within 5% of
+// the least over the first eight counts from one full round on: at C = 80 (20 quads on
+// 32 slots) one range leaves 12 slots idle, three fill 60 of 64.
 struct MaceShape {
     int n_quads, ranges_per_xcd, n_workers;
     unsigned grid;
@@ -950,7 +1043,13 @@ static int mace_shape(K kernel, int waves, int C, MaceShape* sh) {
         occ = 1;
     const int per_xcd = std::max(1, mace_cu_count() / 8);
     sh->n_quads = mace_quads(C);
-    sh->ranges_per_xcd = std::max(1, per_xcd * occ / sh->n_quads);
+    const int slots = per_xcd * occ, first = std::max(1, slots / sh->n_quads);
+    const int last = std::min(first + 7, kMaceMaxWorkers / (8 * waves));
+    auto cost = [&](int r) { return (double)ceil_div((int64_t)r * sh->n_quads, slots) / r; };
+    int best = first;
+    for (int r = first + 1; r <= last; ++r)
+        if (cost(r) < 0.95 * cost(best)) best = r;
+    sh->ranges_per_xcd = best;
     sh->n_workers = 8 * sh->ranges_per_xcd * waves;
     if (sh->n_workers > kMaceMaxWorkers) return BM_ERR_ARG;
     sh->grid = (unsigned)(8 * sh->ranges_per_xcd * sh->n_quads);
