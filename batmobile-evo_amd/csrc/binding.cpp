@@ -188,11 +188,13 @@ torch::Tensor tensor_product(const torch::Tensor& input1, const torch::Tensor& i
     torch::Tensor out = torch::empty({N, C_out, 16}, f32_like(input1));
     if (N == 0) return out;
     const c10::DeviceGuard guard(input1.device());
-    check_status(batteries_tensor_product_l3(cptr<float>(input1, "input1"),
-                                             cptr<float>(input2, "input2"),
-                                             cptr<float>(weights, "weights"),
-                                             mptr<float>(out, "output"), N, (int)C_in, (int)C_out,
-                                             current_stream(input1)),
+    const size_t wsb = batteries_tensor_product_l3_workspace_bytes(N, (int)C_in, (int)C_out);
+    torch::Tensor ws;
+    if (wsb) ws = torch::empty({(int64_t)((wsb + 3) / 4)}, f32_like(input1));
+    check_status(batteries_tensor_product_l3_ws(
+                     cptr<float>(input1, "input1"), cptr<float>(input2, "input2"),
+                     cptr<float>(weights, "weights"), mptr<float>(out, "output"), N, (int)C_in,
+                     (int)C_out, wsb ? ws.data_ptr() : nullptr, wsb, current_stream(input1)),
                  "tensor_product");
     return out;
 }
@@ -267,11 +269,10 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> tensor_product_backward(
     }
     const c10::DeviceGuard guard(input1.device());
     torch::Tensor ws;
-    size_t wsb = 0;
-    if (needs_weights_grad) {  // grad_W partials of the row segments
-        wsb = batteries_tensor_product_backward_workspace_bytes(N, (int)C_in, (int)C_out);
-        ws = torch::empty({(int64_t)((wsb + 3) / 4)}, opt);
-    }
+    // split weights of the mixing kernel, then the grad_W partials of the row segments
+    const size_t wsb = batteries_tensor_product_backward_l3_workspace_bytes(
+        N, (int)C_in, (int)C_out, needs_weights_grad ? 1 : 0);
+    if (wsb) ws = torch::empty({(int64_t)((wsb + 3) / 4)}, opt);
     check_status(batteries_tensor_product_backward_l3(
                      cptr<float>(input1, "input1"), cptr<float>(input2, "input2"),
                      cptr<float>(weights, "weights"), cptr<float>(grad_output, "grad_output"),

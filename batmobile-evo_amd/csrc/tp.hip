@@ -225,8 +225,9 @@ __global__ __launch_bounds__(kTpBlock) void tp_simple_backward_kernel(
 //   gy[n,b]     = sum_{ci,q,a} c * x[n,ci,a] * h[n,ci,q]
 //   gW[p,ci,co] = sum_n sum_{q in p} T[n,ci,q] * g[n,co,out(q)]
 //
-// The three channel contractions (out, h, gW) are GEMMs per slot and run on
-// v_mfma_f32_16x16x4f32 over 16-row tiles; the CG contractions (T, gx, gy) run
+// The three channel contractions (out, h, gW) are GEMMs per slot.  Calls with few rows or
+// no workspace run on v_mfma_f32_16x16x4f32 over 16-row tiles as follows; the others take the
+// mixing kernel further below.  The CG contractions (T, gx, gy) run
 // on the VALU with compile-time coefficients.  Each kernel splits the slots
 // into groups taken by different workgroups, so that a group's
 // outputs are disjoint from the others':
@@ -746,6 +747,371 @@ __global__ __launch_bounds__(512) void tp_weighted_bwd_xy_mfma_kernel(
     }
 }
 
+// ---- channel mixing of many rows: the forward, and grad_input1 / grad_input2 -------
+// One structure serves both.  Z is the operand whose channels are contracted (the
+// forward: input1 over C_in; the backward: grad_output over C_out) and, per path p and
+// component z of its Z side,
+//   h_p[row][i][z] = sum_k W_p[i, k] Z[row][k][z]
+// on the bf16 matrix cores (common.h), after which the CG entries of p are applied on the
+// VALU: out[o] += c y[b] h_p[a], or gx[a] += c y[b] h_p[o] and gy[b] += c x[a] h_p[o].
+// Mixing before the CG contraction keeps Z, 16 values a row and channel, the operand that
+// is split and staged; contracted first, it is 156.
+//
+// Workgroup: 16 rows, 8 waves.  Up to 64 contracted channels of Z sit in LDS as operand
+// fragments sZ[(z * KS + s) * 3 + part][lane] (row lane % 16, channels 32 s + 8 (lane / 16)
+// .. + 7); further channels run chunk by chunk.  A unit is (16-channel tile of i, degree L
+// of the output side): its wave keeps those 2 L + 1 output components in registers and
+// takes the unit's paths in turn.  A pass covers up to four channel tiles; mix_unit_of
+// deals its units so that every SIMD has about the same slots (16, 39, 51 and 50 of the
+// 156 for L = 0..3).  The results meet in LDS (sO) and leave as whole lines: stored from
+// the units, a 64-byte row is written in pieces by four waves (206 of 740 us at 60,013 rows,
+// 64 x 64 channels).  The weights come split, in fragment order, from
+// tp_weighted_pack_kernel (5 us).
+// Bound: MFMA and VALU issue (1872 MFMAs of 16 cycles and, forward, 2,800 CG operations per
+// 16 x 16 unit of 64 channels), and the staging and stores that one workgroup per CU does
+// not overlap.  60,000 rows, against the fp32 MFMA kernels above, forward / backward:
+// 64 -> 64 channels 958 -> 469 / 802 -> 692 us, 32 -> 32 493 -> 170 / 447 -> 243,
+// 48 -> 72 1802 -> 584 / 1921 -> 876, 128 -> 8 1631 -> 420 / 1476 -> 792.  Error against
+// 64 bits 1.5e-7 (forward; 2.3e-7 before), 1.9e-7 (backward; the same).
+// ---------------------------------------------------------------------------------
+constexpr int kMixTiles = 4;   // channel tiles of i per pass
+constexpr int kMixWaves = 8;   // two per SIMD (waves w and w + 4)
+
+constexpr int mix_l_in(int p, bool fwd) { return kPathL[p][fwd ? 0 : 2]; }
+constexpr int mix_l_out(int p, bool fwd) { return kPathL[p][fwd ? 2 : 0]; }
+// The paths of a unit of degree L, by degree of the Z side: how many, and the k-th.
+constexpr int mix_unit_paths(int L, bool fwd) {
+    int c = 0;
+    for (int p = 0; p < kNumPaths; ++p) c += mix_l_out(p, fwd) == L;
+    return c;
+}
+constexpr int mix_unit_path(int k, int L, bool fwd) {
+    for (int lz = 0; lz < 4; ++lz)
+        for (int p = 0; p < kNumPaths; ++p)
+            if (mix_l_in(p, fwd) == lz && mix_l_out(p, fwd) == L && k-- == 0) return p;
+    return -1;
+}
+
+// Entry i is the first of its path with its (a, o).
+constexpr bool mix_first_of_pair(int i) {
+    for (int j = kPathEntry[kCG[i].p]; j < i; ++j)
+        if (kCG[j].a == kCG[i].a && kCG[j].o == kCG[i].o) return false;
+    return true;
+}
+
+// Unit u (0 or 1) of wave w in a pass of nt tiles: 4 * tile + L, or -1.  nt = 4: each SIMD
+// has a tile, one wave L = 2 then 0, the other L = 3 then 1; nt = 3: three SIMDs a tile's
+// L = 2 then 0 and L = 3, the fourth the three L = 1; nt = 2: L = 2 and 0, or L = 3 and 1;
+// nt = 1: one each.
+__device__ __forceinline__ int mix_unit_of(int nt, int w, int u) {
+    const int s = w & 3, k = w >> 2;
+    if (nt == 4) return 4 * s + (k == 0 ? 2 - 2 * u : 3 - 2 * u);
+    if (nt == 3) {
+        if (s == 3) return k == 0 ? 4 * u + 1 : (u == 0 ? 9 : -1);
+        return k == 0 ? 4 * s + 2 - 2 * u : (u == 0 ? 4 * s + 3 : -1);
+    }
+    if (u > 0) return -1;
+    if (nt == 2) return 4 * (s & 1) + (k == 0 ? 2 + (s >> 1) : (s >> 1));
+    return k > 0 ? -1 : 3 - s;
+}
+
+// Place of (row, channel i of the pass, component c) in sO: 16-byte rows rotated so that
+// both the units' accesses (16 rows x 4 channels of one component) and the copies' (4
+// channels x 16 components of a row) meet 64 different banks.
+__device__ __forceinline__ int mix_so(int row, int i, int c) {
+    const int rot = (row >> 2) * 4 + ((i >> 2) & 3);
+    return (i * 16 + (row ^ (i & 3))) * 16 + ((c + rot) & 15);
+}
+
+// Weights split beforehand, [path][tile of i][32-channel step][part][lane] (1 KB each, zeros
+// past the channels).  One wave per (path, tile, step).
+template <bool FWD>
+__global__ __launch_bounds__(kTpBlock) void tp_weighted_pack_kernel(const float* __restrict__ w,
+                                                                    v4u* __restrict__ wp, int nk,
+                                                                    int ni, int total) {
+    const int id = blockIdx.x * (kTpBlock / 64) + (threadIdx.x >> 6);
+    if (id >= total) return;  // uniform over the wave
+    const int lane = threadIdx.x & 63, nks = (nk + 31) / 32, nit = (ni + 15) / 16;
+    const int s = id % nks, it = id / nks % nit, p = id / (nks * nit);
+    const int i = it * 16 + (lane & 15), k = 32 * s + 8 * (lane >> 4);
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const bool ok = i < ni && k + j < nk;
+        const int kc = min(k + j, nk - 1), ic = min(i, ni - 1);
+        v[j] = mask0(w[(int64_t)p * nk * ni + (FWD ? (int64_t)kc * ni + ic : (int64_t)ic * nk + kc)], ok);
+    }
+    const Bf3 b = bf16_split8(v);
+    v4u* o = wp + (int64_t)id * 192 + lane;
+    o[0] = b.h;
+    o[64] = b.m;
+    o[128] = b.l;
+}
+
+// One unit over the chunk of Z in sZ: wu = the fragments of path 0 for the unit's tile and
+// chunk, pstep = distance between paths, s1 = of the second step (0: there is
+// none, and Z is zero there).  sO holds the chunks' sums so far (first: the backward's x).
+template <bool FWD, int KS, int L>
+__device__ __forceinline__ void mix_unit(const float* __restrict__ xin, float* yb,
+                                         const v4u* __restrict__ wu, int64_t pstep, int s1,
+                                         bool first, int ct, int it, int ni, int64_t row_c,
+                                         const v4u* sZ, float* sO, float* gyp) {
+    constexpr int A0 = L * L, NA = 2 * L + 1;
+    const int lane = threadIdx.x & 63, g4 = lane >> 4, i16 = lane & 15;
+    float xa[FWD ? 1 : 4][NA], acc[4][NA];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int a = 0; a < NA; ++a) acc[r][a] = 0.0f;
+    if (!FWD || !first) {  // uniform
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int a = 0; a < NA; ++a) {
+                const float v = sO[mix_so(i16, it * 16 + 4 * g4 + r, A0 + a)];
+                if (!first) acc[r][a] = v;
+                if constexpr (!FWD) xa[r][a] = v;
+            }
+    }
+    if constexpr (!FWD) {
+        if (!first) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = ct * 16 + 4 * g4 + r;
+#pragma unroll
+                for (int a = 0; a < NA; ++a)
+                    xa[r][a] = mask0(xin[(row_c * ni + min(i, ni - 1)) * 16 + A0 + a], i < ni);
+            }
+        }
+    }
+    // One path per iteration of a loop that is not unrolled: each is a basic block of its
+    // own, so that instruction selection cannot mix the paths' MFMAs and CG terms (in one
+    // block they spill).  The next path's weights are in flight meanwhile.  y and the
+    // distance of the paths pass through an empty asm, so that the products c y[b] and the
+    // weights' addresses are formed where they are used.
+    constexpr int NP = mix_unit_paths(L, FWD);
+    Bf3 wf[2][KS];
+    auto load = [&](auto pc, int slot) {
+        constexpr int p = decltype(pc)::value;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const v4u* f = wu + p * pstep + (s ? s1 : 0);  // uniform
+            wf[slot][s].h = f[lane];
+            wf[slot][s].m = f[lane + 64];
+            wf[slot][s].l = f[lane + 128];
+        }
+    };
+    constexpr int pf = mix_unit_path(0, L, FWD);  // (named: as an argument it runs at run time)
+    load(std::integral_constant<int, pf>{}, 0);
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < NP; ++k) {
+        float* yk = yb;
+        asm volatile("" : "+v"(yk[0]), "+v"(yk[1]), "+v"(yk[2]), "+v"(yk[3]), "+v"(yk[4]),
+                          "+v"(yk[5]), "+v"(yk[6]), "+v"(yk[7]), "+v"(yk[8]), "+v"(yk[9]),
+                          "+v"(yk[10]), "+v"(yk[11]), "+v"(yk[12]), "+v"(yk[13]),
+                          "+v"(yk[14]), "+v"(yk[15]));
+        asm volatile("" : "+s"(pstep));
+        static_for<NP>([&](auto kk) {
+            constexpr int kc = decltype(kk)::value;
+            if (k == kc) {
+                constexpr int p = mix_unit_path(kc, L, FWD), LZ = mix_l_in(p, FWD);
+                if constexpr (kc + 1 < NP) {
+                    constexpr int pn = mix_unit_path(kc + 1, L, FWD);
+                    load(std::integral_constant<int, pn>{}, (kc + 1) & 1);
+                }
+                const Bf3* a = wf[kc & 1];
+                // Component m + 1's fragments are read while component m's MFMAs run, and
+                // component m - 1's CG terms go between them.
+                constexpr int NM = 2 * LZ + 1;
+                Bf3 b[2][KS];
+                v4f h[2];
+                auto read_b = [&](int m, Bf3* dst) {
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) {
+                        const v4u* f = sZ + ((LZ * LZ + m) * KS + s) * 3 * 64 + lane;
+                        dst[s].h = f[0];
+                        dst[s].m = f[64];
+                        dst[s].l = f[128];
+                    }
+                };
+                auto contract = [&](auto mc) {
+                    constexpr int m = decltype(mc)::value, z = LZ * LZ + m;
+                    static_for<kPathEntry[p + 1] - kPathEntry[p]>([&](auto ee) {
+                        constexpr int i = kPathEntry[p] + decltype(ee)::value;
+                        constexpr CGEntry e = kCG[i];
+                        // the entries of one (a, o) together (611 entries, 541 pairs)
+                        if constexpr ((FWD ? e.a : e.o) == z && mix_first_of_pair(i)) {
+                            constexpr int ai = (FWD ? e.o : e.a) - A0;
+                            float cy = e.c * yk[e.b];
+                            static_for<kPathEntry[p + 1] - 1 - i>([&](auto ff) {
+                                constexpr CGEntry f = kCG[i + 1 + decltype(ff)::value];
+                                if constexpr (f.a == e.a && f.o == e.o) cy = fmaf(f.c, yk[f.b], cy);
+                            });
+                            float sacc = 0.0f;
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                acc[r][ai] = fmaf(cy, h[m & 1][r], acc[r][ai]);
+                                if constexpr (!FWD) sacc = fmaf(xa[r][ai], h[m & 1][r], sacc);
+                            }
+                            if constexpr (!FWD) {
+                                gyp[e.b] = fmaf(e.c, sacc, gyp[e.b]);
+                                static_for<kPathEntry[p + 1] - 1 - i>([&](auto ff) {
+                                    constexpr CGEntry f = kCG[i + 1 + decltype(ff)::value];
+                                    if constexpr (f.a == e.a && f.o == e.o)
+                                        gyp[f.b] = fmaf(f.c, sacc, gyp[f.b]);
+                                });
+                            }
+                        }
+                    });
+                };
+                read_b(0, b[0]);
+                static_for<NM>([&](auto mc) {
+                    constexpr int m = decltype(mc)::value;
+                    if constexpr (m + 1 < NM) read_b(m + 1, b[(m + 1) & 1]);
+                    // the five small products in a chain of their own
+                    v4f hi = v4f{0.f, 0.f, 0.f, 0.f}, lo = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) mfma_bf16x6(a[s], b[m & 1][s], hi, lo);
+                    if constexpr (m > 0) contract(std::integral_constant<int, (m > 0 ? m - 1 : 0)>{});
+                    h[m & 1] = hi + lo;
+                    __builtin_amdgcn_sched_barrier(0);  // one component's fragments ahead
+                });
+                contract(std::integral_constant<int, NM - 1>{});
+            }
+        });
+    }
+    // (through an empty asm: the places in sO are formed again, not kept since the reads)
+    int row = i16, i0 = it * 16 + 4 * g4;
+    asm volatile("" : "+v"(row), "+v"(i0));
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int a = 0; a < NA; ++a) sO[mix_so(row, i0 + r, A0 + a)] = acc[r][a];
+}
+
+// FWD: out = result [n][ni][16].  Backward: out = grad_x and gy = grad_y (either may be
+// null), xin = input1 [n][ni][16].
+template <bool FWD, int KS>
+__global__ __launch_bounds__(64 * kMixWaves) void tp_weighted_mix_kernel(
+    const float* __restrict__ z, const float* __restrict__ xin, const float* __restrict__ y,
+    const v4u* __restrict__ wp, float* __restrict__ out, float* __restrict__ gy, int64_t n,
+    int nk, int ni) {
+    extern __shared__ v4u mix_lds[];
+    v4u* sZ = mix_lds;                                            // 48 KS KB
+    float* sO = reinterpret_cast<float*>(mix_lds + 16 * KS * 3 * 64);  // 16 KB a tile of a pass
+    const int tid = threadIdx.x, nthr = blockDim.x, lane = tid & 63, i16 = lane & 15, g4 = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t row0 = (int64_t)blockIdx.x * kTile;
+    const int rows = (int)min<int64_t>(kTile, n - row0);
+    const int nct = (ni + 15) / 16, nks = (nk + 31) / 32;
+    const int64_t pstep = (int64_t)nct * nks * 192, row_c = row0 + min(i16, rows - 1);
+    float yb[16], gyp[16];
+    load16(y, row_c * 16, yb);  // rows >= n reach discarded outputs
+#pragma unroll
+    for (int k = 0; k < 16; ++k) gyp[k] = 0.0f;
+    for (int c0 = 0; c0 < nct; c0 += kMixTiles) {
+        const int nt = min(kMixTiles, nct - c0), chans = min(16 * nt, ni - 16 * c0);
+        for (int k0 = 0; k0 < nk; k0 += 32 * KS) {
+            if (c0 + k0 > 0) __syncthreads();  // the chunk before, or the pass's results, are read
+            // Z of the 16 rows and 32 KS channels, once if it is one chunk: a thread takes 8
+            // channels x 4 components of a row (zeros past n and nk; clamped, unconditional
+            // loads)
+            if (c0 == 0 || nk > 32 * KS)
+                for (int i = tid; i < 16 * 4 * KS * 4; i += nthr) {
+                    const int zq = i & 3, r = (i >> 2) & 15, oct = i >> 6;
+                    const int k = k0 + 8 * oct;
+                    const float* src = z + (row0 + min(r, rows - 1)) * nk * 16 + 4 * zq;
+                    float4 v[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        v[j] = *reinterpret_cast<const float4*>(src + min(k + j, nk - 1) * 16);
+                    float c[4][8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const bool ok = r < rows && k + j < nk;
+                        c[0][j] = mask0(v[j].x, ok);
+                        c[1][j] = mask0(v[j].y, ok);
+                        c[2][j] = mask0(v[j].z, ok);
+                        c[3][j] = mask0(v[j].w, ok);
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const Bf3 b = bf16_split8(c[q]);
+                        v4u* f = sZ + ((4 * zq + q) * KS + (oct >> 2)) * 3 * 64 + (oct & 3) * 16 + r;
+                        f[0] = b.h;
+                        f[64] = b.m;
+                        f[128] = b.l;
+                    }
+                }
+            // the backward's x of the pass (zeros past n and the channels), in whole lines
+            if constexpr (!FWD)
+                if (k0 == 0) {
+#pragma clang loop unroll(disable)
+                    for (int i0 = tid; i0 < 1024 * nt; i0 += 4 * nthr) {
+                        float4 v[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const int i = i0 + k * nthr, r = (i >> 2) & 15, c = 4 * (i >> 8) + ((i >> 6) & 3);
+                            v[k] = *reinterpret_cast<const float4*>(
+                                xin + ((row0 + min(r, rows - 1)) * ni + 16 * c0 + min(c, chans - 1)) * 16 +
+                                4 * (i & 3));
+                        }
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const int i = i0 + k * nthr, r = (i >> 2) & 15, c = 4 * (i >> 8) + ((i >> 6) & 3);
+                            if (i >= 1024 * nt) continue;
+                            const bool ok = r < rows && c < chans;
+                            float* o = sO;
+                            o[mix_so(r, c, 4 * (i & 3))] = mask0(v[k].x, ok);
+                            o[mix_so(r, c, 4 * (i & 3) + 1)] = mask0(v[k].y, ok);
+                            o[mix_so(r, c, 4 * (i & 3) + 2)] = mask0(v[k].z, ok);
+                            o[mix_so(r, c, 4 * (i & 3) + 3)] = mask0(v[k].w, ok);
+                        }
+                    }
+                }
+            __syncthreads();
+            const int s1 = KS > 1 && k0 / 32 + 1 < nks ? 192 : 0;
+#pragma clang loop unroll(disable)
+            for (int u = 0; u < 2; ++u) {
+                const int unit = mix_unit_of(nt, wv, u);
+                if (unit < 0) continue;
+                const int it = unit >> 2, ct = c0 + it;
+                const v4u* wu = wp + ((int64_t)ct * nks + k0 / 32) * 192;
+                switch (unit & 3) {
+                    case 0: mix_unit<FWD, KS, 0>(xin, yb, wu, pstep, s1, k0 == 0, ct, it, ni, row_c, sZ, sO, gyp); break;
+                    case 1: mix_unit<FWD, KS, 1>(xin, yb, wu, pstep, s1, k0 == 0, ct, it, ni, row_c, sZ, sO, gyp); break;
+                    case 2: mix_unit<FWD, KS, 2>(xin, yb, wu, pstep, s1, k0 == 0, ct, it, ni, row_c, sZ, sO, gyp); break;
+                    default: mix_unit<FWD, KS, 3>(xin, yb, wu, pstep, s1, k0 == 0, ct, it, ni, row_c, sZ, sO, gyp); break;
+                }
+            }
+        }
+        __syncthreads();
+        if (out)
+            for (int r = wv; r < rows; r += nthr >> 6) {
+                float* o = out + ((row0 + r) * ni + 16 * c0) * 16 + lane;
+#pragma unroll 4
+                for (int q = 0; q < 4 * nt; ++q) {
+                    const int c = 4 * q + (lane >> 4);
+                    const float v = sO[mix_so(r, c, lane & 15)];
+                    if (c < chans) o[64 * q] = v;
+                }
+            }
+    }
+    if (FWD || !gy) return;  // uniform over the workgroup
+    // grad_y: the waves' partials in sZ, summed in a fixed order
+    float* sRed = reinterpret_cast<float*>(sZ);  // [wave][g][row][16]
+#pragma unroll
+    for (int k = 0; k < 16; ++k) sRed[((wv * 4 + g4) * 16 + i16) * 16 + k] = gyp[k];
+    __syncthreads();
+    for (int i = tid; i < rows * 16; i += nthr) {
+        float sum = 0.0f;
+        for (int v = 0; v < nthr / 64; ++v)
+#pragma unroll
+            for (int gg = 0; gg < 4; ++gg) sum += sRed[(v * 4 + gg) * 256 + i];
+        gy[row0 * 16 + i] = sum;
+    }
+}
+
 // ---- backward: grad_W partials over row segments ----------------------------
 // Workgroup: one row segment x 16 input channels x one l1 group x 64 output
 // channels (wave w: co0 .. co0+15).  Per 16-row chunk: thread t builds T for
@@ -1013,6 +1379,46 @@ static int64_t bwd_xy_pairs(int64_t tiles) {
     return ceil_div(tiles, 2);
 }
 
+// The mixing kernel serves a call when the caller's workspace has room for the split
+// weights.  Forward: from kMixRows rows on; below, the weights' split and workgroups of 16
+// rows x all output channels (fewer than the compute units) cost more than they save (32 ->
+// 64 channels: 20.1 -> 23.5 us at 1,400 rows, 29.6 -> 24.4 at 3,072).  With many more output
+// than input channels the CG terms, here per output channel, weigh more: 8 -> 128 channels
+// 37.8 -> 40.8 us at 3,072 rows, 115 -> 111 at 10,000.  Backward: always (32 -> 64 channels
+// 35.9 -> 25.4 us at 100 rows, 462 -> 419 at 60,000; 48 -> 72: 1921 -> 876).
+constexpr int64_t kMixRows = 3072, kMixRowsWide = 8192;
+static bool mix_forward_rows(int64_t n, int cin, int cout) {
+    return n >= (cout > 8 * cin ? kMixRowsWide : kMixRows);
+}
+static size_t mix_packed_bytes(int nk, int ni) {
+    return (size_t)kNumPaths * ceil_div(ni, 16) * ceil_div(nk, 32) * 192 * sizeof(v4u);
+}
+static bool mix_serves(int nk, int ni, const void* workspace, size_t bytes) {
+    return workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
+           (int64_t)kNumPaths * nk * ni * 4 <= INT32_MAX && bytes >= mix_packed_bytes(nk, ni);
+}
+template <bool FWD>
+static int mix_launch(const float* z, const float* xin, const float* y, const float* w,
+                      void* workspace, float* out, float* gy, int64_t n, int nk, int ni,
+                      hipStream_t stream) {
+    v4u* wp = static_cast<v4u*>(workspace);
+    const int total = kNumPaths * (int)(ceil_div(ni, 16) * ceil_div(nk, 32));
+    tp_weighted_pack_kernel<FWD><<<(unsigned)ceil_div(total, kTpBlock / 64), kTpBlock, 0, stream>>>(
+        w, wp, nk, ni, total);
+    const unsigned grid = (unsigned)ceil_div(n, kTile);
+    // one channel tile has four units; LDS by the tiles of a pass
+    const int tiles = std::min<int>(kMixTiles, (int)ceil_div(ni, 16));
+    const int threads = 64 * (tiles == 1 ? 4 : kMixWaves);
+    const size_t lds = (nk <= 32 ? 1 : 2) * (48u << 10) + tiles * (16u << 10);
+    if (nk <= 32)
+        tp_weighted_mix_kernel<FWD, 1><<<grid, threads, lds, stream>>>(z, xin, y, wp, out, gy, n,
+                                                                       nk, ni);
+    else
+        tp_weighted_mix_kernel<FWD, 2><<<grid, threads, lds, stream>>>(z, xin, y, wp, out, gy, n,
+                                                                       nk, ni);
+    return (int)hipGetLastError();
+}
+
 // Row segments of the grad_W reduction: a fixed function of (N, C_in, C_out),
 // not of the device, so results are the same on every GPU.  The grid
 // (segments x input-channel tiles x output-channel blocks x 3 groups) is sized
@@ -1081,18 +1487,41 @@ extern "C" int batteries_tensor_product_simple_backward_l3(const float* input1,
 // larger N runs as consecutive launches over row ranges.
 constexpr int64_t kFwdMaxRowsPerLaunch = int64_t(1) << 24;
 
+// Bytes that let batteries_tensor_product_l3_ws take the mixing kernel (0: it would not).
+extern "C" size_t batteries_tensor_product_l3_workspace_bytes(int64_t N, int C_in, int C_out) {
+    if (C_in <= 0 || C_out <= 0 || !mix_forward_rows(N, C_in, C_out)) return 0;
+    return mix_packed_bytes(C_in, C_out);
+}
+
 extern "C" int batteries_tensor_product_l3(const float* input1, const float* input2,
                                            const float* weights, float* output, int64_t N,
                                            int C_in, int C_out, hipStream_t stream) {
+    return batteries_tensor_product_l3_ws(input1, input2, weights, output, N, C_in, C_out, nullptr,
+                                          0, stream);
+}
+
+extern "C" int batteries_tensor_product_l3_ws(const float* input1, const float* input2,
+                                              const float* weights, float* output, int64_t N,
+                                              int C_in, int C_out, void* workspace,
+                                              size_t workspace_bytes, hipStream_t stream) {
     if (N < 0 || C_in <= 0 || C_out <= 0) return BM_ERR_ARG;
     if (N == 0) return BM_OK;
     if (ceil_div(C_out, 64) > 65535) return BM_ERR_ARG;
     if ((int64_t)kNumPaths * C_in * C_out * 4 > INT32_MAX) return BM_ERR_ARG;  // W via 32-bit offsets
     if ((reinterpret_cast<uintptr_t>(input1) | reinterpret_cast<uintptr_t>(output)) & 15)
         return BM_ERR_ARG;
+    const bool mix = mix_forward_rows(N, C_in, C_out) &&
+                     mix_serves(C_in, C_out, workspace, workspace_bytes);
     const int halves = C_in > 16 ? 2 : 1;  // input-channel chunks split over two wave halves
     for (int64_t r0 = 0; r0 < N; r0 += kFwdMaxRowsPerLaunch) {
         const int64_t rows = std::min(kFwdMaxRowsPerLaunch, N - r0);
+        if (mix) {
+            const int rc = mix_launch<true>(input1 + r0 * C_in * 16, nullptr, input2 + r0 * 16,
+                                            weights, workspace, output + r0 * C_out * 16, nullptr,
+                                            rows, C_in, C_out, stream);
+            if (rc != BM_OK) return rc;
+            continue;
+        }
         const int64_t ntile = ceil_div(rows, kTile);
         // (row tile, group) pairs: tiles rounded up to 8, four groups each
         dim3 grid((unsigned)(ceil_div(ntile, 8) * 8 * kFwdGroups), (unsigned)ceil_div(C_out, 64), 1);
@@ -1114,14 +1543,31 @@ extern "C" size_t batteries_tensor_product_backward_workspace_bytes(int64_t N, i
            sizeof(float);
 }
 
-// The weighted backward on a given workspace (gw_part: the grad_W partials, at least
-// batteries_tensor_product_backward_workspace_bytes when grad_weights is computed).
+// The same with room for the mixing kernel's split weights (which share the space: they are
+// read before the partials are written).
+extern "C" size_t batteries_tensor_product_backward_l3_workspace_bytes(int64_t N, int C_in,
+                                                                       int C_out,
+                                                                       int with_weights) {
+    if (N <= 0 || C_in <= 0 || C_out <= 0) return 0;
+    const size_t gw =
+        with_weights ? batteries_tensor_product_backward_workspace_bytes(N, C_in, C_out) : 0;
+    return std::max(gw, mix_packed_bytes(C_out, C_in));
+}
+
+// The weighted backward on a given workspace (null or `bytes` bytes; at least
+// batteries_tensor_product_backward_workspace_bytes when grad_weights is computed).  It
+// holds the split weights of the mixing kernel, then the grad_W partials.
 static int tp_backward_run(const float* input1, const float* input2, const float* weights,
                            const float* grad_output, float* grad_input1, float* grad_input2,
-                           float* grad_weights, int64_t N, int C_in, int C_out, float* gw_part,
-                           hipStream_t stream) {
+                           float* grad_weights, int64_t N, int C_in, int C_out, void* workspace,
+                           size_t bytes, hipStream_t stream) {
+    float* gw_part = static_cast<float*>(workspace);
     if (grad_input1 || grad_input2) {
-        if (C_out <= 128 && (int64_t)kNumPaths * C_in * C_out * 4 <= INT32_MAX) {
+        if (mix_serves(C_out, C_in, workspace, bytes)) {
+            const int rc = mix_launch<false>(grad_output, input1, input2, weights, workspace,
+                                             grad_input1, grad_input2, N, C_out, C_in, stream);
+            if (rc != BM_OK) return rc;
+        } else if (C_out <= 128 && (int64_t)kNumPaths * C_in * C_out * 4 <= INT32_MAX) {
             // one wave per (path group, 16-channel tile), at most 8 per workgroup;
             // two row tiles on 8 waves when that spreads the units evenly over the SIMDs
             const int nct = (int)ceil_div(C_in, 16);
@@ -1217,7 +1663,8 @@ extern "C" int batteries_tensor_product_backward_l3(
     const size_t need = batteries_tensor_product_backward_workspace_bytes(N, C_in, C_out);
     if (grad_weights && (!workspace || workspace_bytes < need)) return BM_ERR_WORKSPACE;
     return tp_backward_run(input1, input2, weights, grad_output, grad_input1, grad_input2,
-                           grad_weights, N, C_in, C_out, static_cast<float*>(workspace), stream);
+                           grad_weights, N, C_in, C_out, workspace, workspace ? workspace_bytes : 0,
+                           stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1266,11 +1713,13 @@ extern "C" int batteries_tensor_product_backward_l3_noalloc(
         return BATMOBILE_HIP_ERR_SCRATCH;
     const int rc = tp_backward_check(input1, grad_output, grad_weights, N, C_in, C_out, stream);
     if (rc != BM_OK) return rc == 1 ? BM_OK : rc;
+    // (without grad_weights the array is not touched: such calls may overlap)
     float* part = nullptr;
     if (grad_weights) {
         const int e = scratch_address(&part);
         if (e != BM_OK) return e;
     }
     return tp_backward_run(input1, input2, weights, grad_output, grad_input1, grad_input2,
-                           grad_weights, N, C_in, C_out, part, stream);
+                           grad_weights, N, C_in, C_out, part,
+                           part ? BATMOBILE_HIP_NOALLOC_SCRATCH_BYTES : 0, stream);
 }

@@ -93,7 +93,19 @@ int batteries_tensor_product_simple_backward_l3(const float* input1, const float
 int batteries_tensor_product_l3(const float* input1, const float* input2, const float* weights,
                                 float* output, int64_t N, int C_in, int C_out, hipStream_t stream);
 
-/* Workspace for batteries_tensor_product_backward_l3 with grad_weights != NULL. */
+/* The same with a workspace: with room for batteries_tensor_product_l3_workspace_bytes (0
+ * for calls of few rows) the weights are split into the matrix cores' operands once for
+ * all workgroups.  workspace may be NULL; results agree to rounding. */
+size_t batteries_tensor_product_l3_workspace_bytes(int64_t N, int C_in, int C_out);
+int batteries_tensor_product_l3_ws(const float* input1, const float* input2, const float* weights,
+                                   float* output, int64_t N, int C_in, int C_out, void* workspace,
+                                   size_t workspace_bytes, hipStream_t stream);
+
+/* Least workspace for batteries_tensor_product_backward_l3 with grad_weights != NULL (none is
+ * needed without), and the workspace with which it is fastest (with_weights: grad_weights is
+ * wanted). */
+size_t batteries_tensor_product_backward_l3_workspace_bytes(int64_t N, int C_in, int C_out,
+                                                            int with_weights);
 size_t batteries_tensor_product_backward_workspace_bytes(int64_t N, int C_in, int C_out);
 
 /* Exact adjoint of batteries_tensor_product_l3.  Any of grad_input1 [N,C_in,16],

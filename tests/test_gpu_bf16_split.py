@@ -1,4 +1,5 @@
-"""fp32 products on the bf16 matrix cores (three-part operands, six products): the MACE
+"""fp32 products on the bf16 matrix cores (three-part operands, six products): the mixing
+kernel of the weighted tensor product at the edges of its tiles, passes and chunks, the MACE
 layer's weights GEMM at channel counts that fill its quads and launch rounds unevenly,
 its error against float64, and infinities in W2."""
 import numpy as np
@@ -6,6 +7,7 @@ import pytest
 import torch
 
 from oracle import mace as om
+from oracle import tp as otp
 
 from helpers import gen, periodic_box
 
@@ -55,3 +57,54 @@ def test_infinite_weight_stays_infinite(bm, dev):
     # destinations with one edge: +-inf, the sign of h[5] x
     one = deg == 1
     assert torch.isinf(out[one, 1, 0]).all()
+
+
+def _product_inputs(n, ci, co, seed):
+    x = torch.randn(n, ci, 16, generator=gen(seed))
+    y = torch.randn(n, 16, generator=gen(seed + 1))
+    w = torch.randn(34, ci, co, generator=gen(seed + 2)) / ci ** 0.5
+    g = torch.randn(n, co, 16, generator=gen(seed + 3))
+    return x, y, w, g
+
+
+# rows: one below and at the forward's line, a last tile of 15 rows, single rows; channels:
+# parts of a tile, 1 to 4 tiles of a pass and past it, contracted channels of one 32-step, two,
+# a partial second, and past one chunk of 64
+@pytest.mark.parametrize("n,ci,co", [(3071, 8, 8), (3072, 1, 3), (3087, 33, 17), (3073, 64, 65),
+                                     (3072, 20, 130), (3088, 130, 20), (3072, 72, 48), (1, 40, 96),
+                                     (17, 48, 150), (8200, 4, 40)])
+def test_mixing_kernel(bm, dev, n, ci, co):
+    x, y, w, g = _product_inputs(n, ci, co, 51)
+    out = bm.tensor_product(x.to(dev), y.to(dev), w.to(dev)).cpu().double().numpy()
+    gx, gy, gw = bm.tensor_product_backward(x.to(dev), y.to(dev), w.to(dev), g.to(dev))
+    only = bm.tensor_product_backward(x.to(dev), y.to(dev), w.to(dev), g.to(dev), False, True, False)
+    assert torch.equal(only[1], gy)
+    rows = np.unique(np.r_[:20, max(0, n // 2 - 8):n // 2, max(0, n - 20):n])
+    rows = rows[rows < n]
+    xs, ys, gs = (t[rows].double().numpy() for t in (x, y, g))
+    want = otp.tensor_product(xs, ys, w.double().numpy())
+    wx, wy, _ = otp.tensor_product_backward(xs, ys, w.double().numpy(), gs)
+    # sums of up to 34 * 130 fp32 terms: a few 2^-24 times the square root of their number
+    for got, ref in ((out[rows], want), (gx.cpu().double().numpy()[rows], wx),
+                     (gy.cpu().double().numpy()[rows], wy)):
+        assert np.linalg.norm(got - ref) <= 1e-6 * np.linalg.norm(ref)
+
+
+def test_mixing_kernel_infinities(bm, dev):
+    """inf in component 0 of one row's channel reaches that row's outputs through the paths
+    (0, l, l) only, as sign(W y) inf, and no other row; the same for an infinite weight."""
+    n, ci, co = 3072, 40, 24
+    x, y, w, _ = _product_inputs(n, ci, co, 61)
+    x[5, 3, 0] = float("inf")
+    out = bm.tensor_product(x.to(dev), y.to(dev), w.to(dev)).cpu()
+    l = torch.tensor([0] + [1] * 3 + [2] * 5 + [3] * 7)
+    sign = torch.sign(w[l, 3, :].T * y[5])          # path l is (0, l, l)
+    assert torch.equal(out[5], sign * float("inf"))
+    keep = torch.arange(n) != 5
+    assert torch.isfinite(out[keep]).all()
+    x[5, 3, 0] = 1.0
+    w[0, 7, 11] = float("-inf")
+    out = bm.tensor_product(x.to(dev), y.to(dev), w.to(dev)).cpu()
+    assert torch.equal(out[:, 11, 0], -torch.sign(x[:, 7, 0] * y[:, 0]) * float("inf"))
+    out[:, 11, 0] = 0.0
+    assert torch.isfinite(out).all()
