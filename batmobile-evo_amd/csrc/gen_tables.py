@@ -140,6 +140,76 @@ def sh_polynomials(lmax=LMAX_TP):
     return polys
 
 
+def _sh_values(r, lmax=LMAX_TP):
+    """Y of the rows of r by the recurrence, a list of [n, 2l+1] per degree."""
+    ys = [np.ones((r.shape[0], 1))]
+    for l, terms in enumerate(sh_recurrence()[:lmax]):
+        y = np.zeros((r.shape[0], 2 * l + 3))
+        for (M, m, j, c) in terms:
+            y[:, M] += c * ys[-1][:, m] * r[:, j]
+        ys.append(y)
+    return ys
+
+
+def _wigner(rot, lmax=LMAX_TP):
+    """D_l with Y_l(R r) = D_l Y_l(r), l = 0..lmax."""
+    r = np.random.default_rng(5).normal(size=(60, 3))
+    return [np.linalg.lstsq(a, b, rcond=None)[0].T
+            for a, b in zip(_sh_values(r, lmax), _sh_values(r @ rot.T, lmax))]
+
+
+def tilt_polynomials(lmax=LMAX_TP):
+    """t[l, i, j, k]: D_l(i, j) = sum_k t c^(d-k) s^k of the rotation about x that takes the
+    unit vector (0, c, s) to the polar axis y.  d = l for the components even in x (index
+    l .. 2l), l - 1 for the odd ones (0 .. l - 1), which do not mix with them."""
+    t = np.zeros((lmax + 1, 2 * lmax + 1, 2 * lmax + 1, lmax + 1))
+    th = np.linspace(0.1, 6.0, 25)
+    ds = [_wigner(np.array([[1, 0, 0], [0, np.cos(a), np.sin(a)], [0, -np.sin(a), np.cos(a)]]))
+          for a in th]
+    for l in range(lmax + 1):
+        for i in range(2 * l + 1):
+            for j in range(2 * l + 1):
+                v = np.array([d[l][i, j] for d in ds])
+                if (i < l) != (j < l):
+                    assert np.abs(v).max() < 1e-10
+                    continue
+                deg = l if i >= l else l - 1
+                basis = np.stack([np.cos(th) ** (deg - k) * np.sin(th) ** k
+                                  for k in range(deg + 1)], 1)
+                x, *_ = np.linalg.lstsq(basis, v, rcond=None)
+                assert np.abs(basis @ x - v).max() < 1e-10
+                t[l, i, j, :deg + 1] = np.where(np.abs(x) > 1e-9, x, 0.0)
+    for l in range(lmax + 1):
+        for i in range(2 * l + 1):
+            for j in range(i):
+                a, b = t[l, i, j], t[l, j, i]
+                assert np.abs(a - b).max() < 1e-9 or np.abs(a + b).max() < 1e-9
+    return t
+
+
+def rotation_generators():
+    """J[axis, i, j] (axes x and z, components 0..15): Y(r + w e_axis x r) = Y + w J Y."""
+    out = np.zeros((2, 16, 16))
+    h = 1e-3
+    for n, axis in enumerate((0, 2)):
+        e = np.zeros(3)
+        e[axis] = 1.0
+        k = np.array([[0, -e[2], e[1]], [e[2], 0, -e[0]], [-e[1], e[0], 0]])
+
+        def rot(a):
+            return np.eye(3) + np.sin(a) * k + (1 - np.cos(a)) * (k @ k)
+
+        for l in range(4):
+            # D of the small rotations is exp(a J): J from the odd part, Richardson twice
+            d = [( _wigner(rot(a))[l] - _wigner(rot(-a))[l]) / (2 * a) for a in (h, 2 * h, 4 * h)]
+            r1 = (4 * d[0] - d[1]) / 3, (4 * d[1] - d[2]) / 3
+            j = (16 * r1[0] - r1[1]) / 15
+            s = slice(l * l, (l + 1) ** 2)
+            out[n, s, s] = np.where(np.abs(j) > 1e-6, j, 0.0)
+    assert np.abs(out + out.transpose(0, 2, 1)).max() < 1e-8
+    return out
+
+
 def _flit(v):
     return repr(float(v)) + "f" if "e" in repr(float(v)) or "." in repr(float(v)) else repr(float(v)) + ".0f"
 
@@ -235,6 +305,30 @@ def render():
     w(f"constexpr int kSHMonoCount = {len(mono)};")
     w("constexpr SHMono kSHMono[kSHMonoCount] = {")
     w(",\n".join(f"    {{{k}, {e[0]}, {e[1]}, {e[2]}, {_flit(v)}}}" for k, e, v in mono))
+    w("};")
+    w("")
+    tl = tilt_polynomials()
+    w("// Rotation about x that takes the unit vector (0, c, s) to y: its matrix in the")
+    w("// components of degree l, D_l(i, j) = sum_k kTilt[l][i][j][k] c^(d-k) s^k with d = l for")
+    w("// i, j >= l, l - 1 for i, j < l, and 0 between them.")
+    w("constexpr float kTilt[4][7][7][4] = {")
+    w(",\n".join("    {" + ", ".join(
+        "{" + ", ".join("{" + ", ".join(_flit(v) for v in tl[l, i, j]) + "}" for j in range(7)) + "}"
+        for i in range(7)) + "}" for l in range(4)))
+    w("};")
+    w("")
+    gen = rotation_generators()
+    w("// Generators of rotations about x and z, kGen[axis][i][j] with i < j (antisymmetric):")
+    w("// Y(r + w e x r) = Y + w J Y.")
+    terms = [(n, i, j, gen[n, i, j]) for n in range(2) for i in range(16) for j in range(i + 1, 16)
+             if gen[n, i, j] != 0.0]
+    w("struct GenTerm {")
+    w("    int axis, i, j;  // axis 0: x, 1: z")
+    w("    float v;")
+    w("};")
+    w(f"constexpr int kNumGen = {len(terms)};")
+    w("constexpr GenTerm kGen[kNumGen] = {")
+    w(",\n".join(f"    {{{n}, {i}, {j}, {_flit(v)}}}" for n, i, j, v in terms))
     w("};")
     w("")
     w("}  // namespace bmhip")

@@ -16,14 +16,14 @@
 // (557 kflop per edge at C = 128).  One kernel per pass runs it on the bf16 matrix
 // cores (each fp32 operand as three bf16 parts, six products: common.h) and
 // consumes each tile of per-edge weights R straight from the accumulators in
-// the channel-wise CG product on the VALU (611 products with a coefficient,
-// 256 bilinear products and 156 path weightings per edge and channel), so R
-// (26 GB at configs[4]) never reaches memory.  The backward runs the same
-// tiles with the MLP's transpose GEMM on MFMA fed by the path gradients, and
-// ends in per-edge position gradients; forces are gathered per atom through
+// the channel-wise CG product on the VALU, formed in the frame of the edge
+// (aligned.h: about 340 operations per edge and channel against 1023), so R
+// (26 GB at configs[4]) never reaches memory.  The backward forms R and its
+// derivative along the edge length by the same GEMM, contracts both with the
+// incoming gradient in the same frame, and ends in per-edge position gradients; forces are gathered per atom through
 // the reverse-edge map of the symmetric edge list.  Every sum runs in a fixed
 // order (deterministic, no atomics).
-#include "common.h"
+#include "aligned.h"
 #include "batmobile_hip.h"
 
 namespace bmhip {
@@ -161,176 +161,6 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
     }
 }
 
-// One past the last path of the (l1, l2) block that starts at path p0 (the path
-// order is l1 outer, l2, l_out inner, so a block's paths are consecutive).
-constexpr int block_end(int p0) {
-    int p = p0;
-    while (p < kNumPaths && kPathL[p][0] == kPathL[p0][0] && kPathL[p][1] == kPathL[p0][1]) ++p;
-    return p;
-}
-constexpr int path_slot(int p) { return p < kNumPaths ? kPathSlot[p] : kNumSlots; }
-
-// Entry e of path p is the first of its path to write its output slot (when the
-// entries are taken component a ascending, then in table order): the slot's
-// accumulator starts from that term instead of from zero.
-constexpr bool first_slot_write(int p, int e) {
-    const CGEntry& x = kCG[kPathEntry[p] + e];
-    for (int i = kPathEntry[p]; i < kPathEntry[p + 1]; ++i) {
-        const CGEntry& y = kCG[i];
-        if (y.q == x.q && (y.a < x.a || (y.a == x.a && i < kPathEntry[p] + e))) return false;
-    }
-    return true;
-}
-// The same for the input-2 component b (the backward's per-path sums over b).
-constexpr bool first_b_write(int p, int e) {
-    const CGEntry& x = kCG[kPathEntry[p] + e];
-    for (int i = kPathEntry[p]; i < kPathEntry[p + 1]; ++i) {
-        const CGEntry& y = kCG[i];
-        if (y.b == x.b && (y.a < x.a || (y.a == x.a && i < kPathEntry[p] + e))) return false;
-    }
-    return true;
-}
-// every output slot and every component b of every path has an entry (so each
-// accumulator is written before it is read)
-constexpr bool every_slot_and_b_written() {
-    for (int p = 0; p < kNumPaths; ++p) {
-        const int lo = kPathL[p][2], l2 = kPathL[p][1];
-        for (int o = lo * lo; o < (lo + 1) * (lo + 1); ++o) {
-            bool f = false;
-            for (int i = kPathEntry[p]; i < kPathEntry[p + 1]; ++i) f = f || kCG[i].o == o;
-            if (!f) return false;
-        }
-        for (int b = l2 * l2; b < (l2 + 1) * (l2 + 1); ++b) {
-            bool f = false;
-            for (int i = kPathEntry[p]; i < kPathEntry[p + 1]; ++i) f = f || kCG[i].b == b;
-            if (!f) return false;
-        }
-    }
-    return true;
-}
-static_assert(every_slot_and_b_written(), "a path output or input-2 component without entries");
-
-// x * c with c a compile-time coefficient (no multiply for c = 1)
-template <int P, int E>
-__device__ __forceinline__ float cg_times(float x) {
-    constexpr float c = kCG[kPathEntry[P] + E].c;
-    if constexpr (c == 1.0f) return x;
-    else return c * x;
-}
-
-// f(P0, P1) for every (l1, l2) block [P0, P1) of paths, in path order.
-template <int P0, typename F>
-__device__ __forceinline__ void for_blocks(F&& f) {
-    if constexpr (P0 < kNumPaths) {
-        constexpr int P1 = block_end(P0);
-        f(std::integral_constant<int, P0>{}, std::integral_constant<int, P1>{});
-        for_blocks<P1>(f);
-    }
-}
-
-// T_p[o] = sum over the entries (a, b, o) of p of c x[a] Y[b], for the paths of
-// the (l1, l2) block [P0, P1), with each product x[a] Y[b] formed once for the
-// block (256 products per edge and channel over all blocks, against one
-// product c Y[b] per distinct (c, b) when the paths are taken one by one).
-// consume(p, tq) receives T_p (2 l_out + 1 values) of every path of the block.
-template <int P0, int P1, typename F>
-__device__ __forceinline__ void block_products(const float* Y, const float* xs, F&& consume) {
-    constexpr int L1 = kPathL[P0][0], L2 = kPathL[P0][1];
-    constexpr int S0 = kPathSlot[P0], NT = path_slot(P1) - S0;
-    float t[NT];  // each written first by its slot's first term
-    static_for<2 * L1 + 1>([&](auto ia) {
-        constexpr int a = L1 * L1 + decltype(ia)::value;
-        float xy[2 * L2 + 1];
-#pragma unroll
-        for (int i = 0; i < 2 * L2 + 1; ++i) xy[i] = xs[a] * Y[L2 * L2 + i];
-        static_for<P1 - P0>([&](auto pp) {
-            constexpr int p = P0 + decltype(pp)::value;
-            static_for<kPathEntry[p + 1] - kPathEntry[p]>([&](auto ee) {
-                constexpr int e = decltype(ee)::value;
-                constexpr CGEntry en = kCG[kPathEntry[p] + e];
-                if constexpr (en.a == a) {
-                    if constexpr (first_slot_write(p, e))
-                        t[en.q - S0] = cg_times<p, e>(xy[en.b - L2 * L2]);
-                    else
-                        t[en.q - S0] = fmaf(en.c, xy[en.b - L2 * L2], t[en.q - S0]);
-                }
-            });
-        });
-    });
-    static_for<P1 - P0>([&](auto pp) {
-        constexpr int p = P0 + decltype(pp)::value;
-        consume(std::integral_constant<int, p>{}, t + (kPathSlot[p] - S0));
-    });
-}
-
-// m[o] += sum_p R_p T_p[o] over all paths (the forward's per-edge message).
-__device__ __forceinline__ void mace_message(const float* Y, const float* xs, const float* rr,
-                                             float* m) {
-    for_blocks<0>([&](auto b0, auto b1) {
-        block_products<decltype(b0)::value, decltype(b1)::value>(Y, xs, [&](auto pp, const float* tq) {
-            constexpr int p = decltype(pp)::value;
-            constexpr int lo = kPathL[p][2];
-#pragma unroll
-            for (int q = 0; q < 2 * lo + 1; ++q) m[lo * lo + q] = fmaf(rr[p], tq[q], m[lo * lo + q]);
-        });
-    });
-}
-
-// The backward's two contractions of c x[a] Y[b] g[o], by (l1, l_out) blocks:
-// each product x[a] g[o] is formed once (256 per edge and channel) and summed
-// into the block's per-path U_p[b] = sum c x[a] g[o] (one path per l2 within the
-// block, so U is indexed by b); then
-//   gy[b] += R_p U_p[b]                      (the gradient of the pair's Y)
-//   path_grad(p, sum_b Y[b] U_p[b])         (gR_p = g . T_p(x, Y), the weight gradient)
-// so both come from the one set of U (1179 operations per edge and channel against
-// 2046 with T_p formed for gR_p separately).
-template <typename F>
-__device__ __forceinline__ void mace_grad_y(const float* xs, const float* g, const float* Y,
-                                            const float* rr, float* gy, F&& path_grad) {
-    static_for<4>([&](auto l1c) {
-        constexpr int L1 = decltype(l1c)::value;
-        static_for<4>([&](auto loc) {
-            constexpr int LO = decltype(loc)::value;
-            float U[16];  // U[b] written first by its first term (b of the block's paths only)
-            static_for<2 * L1 + 1>([&](auto ia) {
-                constexpr int a = L1 * L1 + decltype(ia)::value;
-                float xg[2 * LO + 1];
-#pragma unroll
-                for (int i = 0; i < 2 * LO + 1; ++i) xg[i] = xs[a] * g[LO * LO + i];
-                static_for<kNumPaths>([&](auto pp) {
-                    constexpr int p = decltype(pp)::value;
-                    if constexpr (kPathL[p][0] == L1 && kPathL[p][2] == LO)
-                        static_for<kPathEntry[p + 1] - kPathEntry[p]>([&](auto ee) {
-                            constexpr int e = decltype(ee)::value;
-                            constexpr CGEntry en = kCG[kPathEntry[p] + e];
-                            if constexpr (en.a == a) {
-                                if constexpr (first_b_write(p, e))
-                                    U[en.b] = cg_times<p, e>(xg[en.o - LO * LO]);
-                                else
-                                    U[en.b] = fmaf(en.c, xg[en.o - LO * LO], U[en.b]);
-                            }
-                        });
-                });
-            });
-            static_for<kNumPaths>([&](auto pp) {
-                constexpr int p = decltype(pp)::value;
-                if constexpr (kPathL[p][0] == L1 && kPathL[p][2] == LO) {
-                    constexpr int l2 = kPathL[p][1];
-                    // gy[b] is first written by the l1 = 0 block of l_out = l2
-#pragma unroll
-                    for (int i = 0; i < 2 * l2 + 1; ++i)
-                        gy[l2 * l2 + i] = L1 == 0 ? rr[p] * U[l2 * l2 + i]
-                                                  : fmaf(rr[p], U[l2 * l2 + i], gy[l2 * l2 + i]);
-                    float gr = Y[l2 * l2] * U[l2 * l2];
-#pragma unroll
-                    for (int i = 1; i < 2 * l2 + 1; ++i) gr = fmaf(Y[l2 * l2 + i], U[l2 * l2 + i], gr);
-                    path_grad(std::integral_constant<int, p>{}, gr);
-                }
-            });
-        });
-    });
-}
-
 __device__ __forceinline__ void load_row16(const float* __restrict__ p, float* v) {
     const float4* q = reinterpret_cast<const float4*>(p);
 #pragma unroll
@@ -397,9 +227,9 @@ __global__ void mace_reverse_edges_kernel(const int64_t* __restrict__ row_ptr,
 //
 // Edges are taken in "positions": the destinations in the given order (a
 // spatial order keeps shared source rows in cache), each destination's edges
-// consecutive and ascending.  A prepass writes per position the unit vector and
-// length, the source and destination, and the radial MLP's hidden layer h
-// [E][64] (the backward also s[E][64], below).
+// consecutive and ascending.  A prepass writes per position the direction, the
+// source and destination, and the radial MLP's hidden layer h [E][64] in three
+// bf16 parts (the backward also the length and s[E][64], below).
 //
 // A workgroup owns one quad of 4 channels c0..c0+3 and keeps that quad's slice
 // of W2 in LDS, split into bf16 parts, as MFMA operand fragments (paths in 9 groups
@@ -411,13 +241,15 @@ __global__ void mace_reverse_edges_kernel(const int64_t* __restrict__ row_ptr,
 // 9 groups: 108 MFMAs of 16 cycles, against 144 of 32 with fp32 MFMAs), and by the
 // accumulator layout lane l = 16 ch + e holds the 34 weights of its own (edge e,
 // channel c0 + ch) pair.  The lane then forms the message of that pair,
-// sum_p R_p T_p(x[src, c], Y(u)), on the VALU.  R never leaves the registers.
+// sum_p R_p T_p(x[src, c], Y(u)), on the VALU (aligned.h).  R never leaves the registers.
 //
 // Bound: VALU + MFMA issue of the SIMD, which overlap little (a probe: 8 FMAs between
 // 16-cycle MFMAs add their whole time with 4 waves per SIMD).  N = 50,000, C = 128,
-// 1.5 M edges: forward kernel 10.5 -> 7.4 ms, backward 17.9 -> 12.6 ms against the fp32
-// MFMA form, the layer's pass 29.0 -> 20.9 ms, its error against 64 bits unchanged
-// (9.8e-7; it comes from the radial basis).
+// 1.5 M edges, forward / backward kernel: fp32 MFMAs and the product by CG entries 10.5 /
+// 17.9 ms; bf16 parts 7.4 / 12.6 ms; product in the edge's frame and the length's
+// derivative by S = s W2 instead of the transpose GEMM 5.1 / 9.7 ms.  The layer's pass
+// with position gradients 29.1 -> 20.9 -> 15.7 ms, its error against 64 bits unchanged
+// (1.0e-6; it comes from the radial basis).
 //
 // Each destination's messages are summed in ascending edge order by one lane
 // after another along the tile (lane e adds lane e - 1's running sum when both
@@ -455,10 +287,12 @@ __device__ __forceinline__ void mace_fill_w2(const float* __restrict__ w2, int C
     }
 }
 
-// The 34 weights of the lane's pair: sA = sW + lane, hb[part * 2 + s] = the part of
-// h[e][32 s + 8 (lane / 16) .. + 7].  The small products of both K steps go first, while
-// the accumulator is small.
-__device__ __forceinline__ void mace_tile_weights(const v4u* sA, const v4u* hb, float* rr) {
+// r_i[p] = sum_k W2[k][p C + c0 + ch] b_i[e][k] of the lane's pair, for NB right-hand
+// sides: sA = sW + lane, b_i[part * 2 + s] = the part of b_i[e][32 s + 8 (lane / 16) .. + 7].
+// The small products of both K steps go first, while the accumulator is small.
+template <int NB>
+__device__ __forceinline__ void mace_tile_weights(const v4u* sA, const v4u* const* b,
+                                                  float* const* r) {
     // the W2 operands are the same for every tile: read them from LDS per tile (an
     // opaque base keeps the compiler from hoisting the reads out of the tile loop)
     int base = 0;
@@ -471,23 +305,22 @@ __device__ __forceinline__ void mace_tile_weights(const v4u* sA, const v4u* hb, 
         for (int s = 0; s < kHSteps; ++s)
 #pragma unroll
             for (int q = 0; q < 3; ++q) a[q * kHSteps + s] = sA[((g * kHSteps + s) * 3 + q) * 64];
-        v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+        v4f acc[NB];
 #pragma unroll
-        for (int s = 0; s < kHSteps; ++s) {
-            acc = mfma_bf16(a[2 * kHSteps + s], hb[s], acc);
-            acc = mfma_bf16(a[s], hb[2 * kHSteps + s], acc);
-            acc = mfma_bf16(a[kHSteps + s], hb[kHSteps + s], acc);
-        }
+        for (int i = 0; i < NB; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
+        constexpr int kA[6] = {2, 0, 1, 1, 0, 0}, kB[6] = {0, 2, 1, 0, 1, 0};  // l h, h l, m m, ...
 #pragma unroll
-        for (int s = 0; s < kHSteps; ++s) {
-            acc = mfma_bf16(a[kHSteps + s], hb[s], acc);
-            acc = mfma_bf16(a[s], hb[kHSteps + s], acc);
-        }
+        for (int t = 0; t < 6; ++t)
 #pragma unroll
-        for (int s = 0; s < kHSteps; ++s) acc = mfma_bf16(a[s], hb[s], acc);
+            for (int s = 0; s < kHSteps; ++s)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (4 * g + j < kNumPaths) rr[4 * g + j] = acc[j];
+                for (int i = 0; i < NB; ++i)
+                    acc[i] = mfma_bf16(a[kA[t] * kHSteps + s], b[i][kB[t] * kHSteps + s], acc[i]);
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (4 * g + j < kNumPaths) r[i][4 * g + j] = acc[i][j];
         __builtin_amdgcn_sched_barrier(0);  // one group's fragments at a time
     });
 }
@@ -502,10 +335,25 @@ __device__ __forceinline__ int dpp_next_i(int v) {  // lane e + 1 of the 16-lane
     return __builtin_amdgcn_update_dpp(0, v, 0x101, 0xF, 0xF, false);
 }
 
+// The frame of edge direction u = (cos f, sin f, c, s).  c = 2 marks an edge of no length:
+// its Y is (1, 0, ...), so only the paths with l2 = 0 act, which need no direction.
+__device__ __forceinline__ void mace_frame(const float4& u, float* r, float* s, AlignedFrame& f) {
+    const bool none = u.z > 1.5f;
+    if (__any(none)) {
+#pragma unroll
+        for (int p = 0; p < kNumPaths; ++p)
+            if (kPathL[p][1] > 0) {
+                r[p] = none ? 0.0f : r[p];
+                s[p] = none ? 0.0f : s[p];
+            }
+    }
+    aligned_frame(u.x, u.y, none ? 1.0f : u.z, u.w, f);
+}
+
 // One tile's per-position operands (pos clamped into the range by the caller).
 struct MaceTileIn {
     v4u hb[3 * kHSteps];
-    float4 u;  // unit vector, length
+    float4 u;  // direction (cos f, sin f, c, s)
     int s, d;
 };
 
@@ -611,17 +459,17 @@ mace_fused_forward_kernel(const float4* __restrict__ u4, const int* __restrict__
             for (int j = 0; j < 3 * kHSteps; ++j) cur.hb[j] = v4u{0, 0, 0, 0};
         }
         float rr[kNumPaths];
-        mace_tile_weights(sA, cur.hb, rr);
+        const v4u* const hp[1] = {cur.hb};
+        float* const rp[1] = {rr};
+        mace_tile_weights<1>(sA, hp, rp);
         // source row of the pair (after the weights: before them its 16 registers spill;
         // the other waves of the SIMD cover its latency)
         float xs[16];
         load_row16(x + ((int64_t)cur.s * C + cc) * 16, xs);
-        float Y[16];
-        sh_forward<3>(cur.u.x, cur.u.y, cur.u.z, Y);
+        AlignedFrame f;
+        mace_frame(cur.u, rr, rr, f);
         float m[16];
-#pragma unroll
-        for (int o = 0; o < 16; ++o) m[o] = 0.0f;
-        mace_message(Y, xs, rr, m);
+        aligned_message(f, xs, rr, m);
         mace_stage_tile(m, e16, kk, sT);
         const int dcur = valid ? cur.d : -1;
         // the next tile's operands (the other waves of the SIMD cover their latency)
@@ -632,66 +480,26 @@ mace_fused_forward_kernel(const float4* __restrict__ u4, const int* __restrict__
     if (carry_d >= 0 && cok) out[((int64_t)carry_d * C + c) * 16 + e16] = acc;
 }
 
-// Place of path p in the order in which mace_grad_y completes the paths (l1, l_out, l2).
-constexpr int grad_slot(int p) {
-    auto key = [](int i) { return (kPathL[i][0] * 4 + kPathL[i][2]) * 4 + kPathL[i][1]; };
-    int n = 0;
-    for (int i = 0; i < kNumPaths; ++i) n += key(i) < key(p) ? 1 : 0;
-    return n;
-}
-struct GradPaths {
-    int path[kNumPaths];
-    constexpr GradPaths() : path{} {
-        for (int p = 0; p < kNumPaths; ++p) path[grad_slot(p)] = p;
-    }
-};
-__constant__ constexpr GradPaths kGradPaths{};
-constexpr int kPOct = (kNumPaths + 7) / 8;           // octets of those places
-constexpr int kW2tFrags = kPOct * 4 * 3;
-
-// The quad's W2 slice as operand fragments of the transpose GEMM, sV[(q * 4 + j) * 3 +
-// part][lane]: row k = 16 j + lane % 16, places 8q .. 8q + 7 of channel c0 + lane / 16.
-__device__ __forceinline__ void mace_fill_w2t(const float* __restrict__ w2, int C, int c0,
-                                              v4u* sV) {
-    for (int i = threadIdx.x; i < kPOct * 4 * 64; i += blockDim.x) {
-        const int lane = i & 63, j = (i >> 6) & 3, q = i >> 8;
-        const int c = c0 + (lane >> 4), k = 16 * j + (lane & 15);
-        float v[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int i = 8 * q + t;
-            v[t] = i < kNumPaths && c < C
-                       ? w2[((int64_t)k * kNumPaths + kGradPaths.path[i]) * C + c] : 0.0f;
-        }
-        const Bf3 b = bf16_split8(v);
-        v4u* f = sV + (q * 4 + j) * 3 * 64 + lane;
-        f[0] = b.h;
-        f[64] = b.m;
-        f[128] = b.l;
-    }
-}
-
-// Backward: per pair, gR_p = sum_o g[d, c, o] T_p[o] feeds the MLP's transpose GEMM
-//   D[k][e] += sum_{ch, p} W2[k][p C + c0 + ch] gR[e, c0 + ch, p]   (K step q = the
-// paths of places 8q .. 8q + 7, of the quad's 4 channels, by 16-row blocks of k: A = W2 from LDS, B = the
-// lane's own 8 gR_p), and gY[b] = sum c x[a] R_p g[o] is summed over the quad's channels.
-// The quad's share of the edge's position gradient,
-//   g_v = g_r u + (g_u - u (u . g_u)) / r,  g_r = sum_k D[k][e] s[e][k],
-//   g_u = SH backward of gY at u,
-// with s[e][k] = silu'(z_k) sum_b W1[b][k] dB_b/dr, goes to gv_part[quad][position].
+// Backward.  The gradient with respect to the length runs back through the MLP as
+//   g_r = sum_{c, p} gR[e, c, p] S[e, c, p],   S = s W2   (= dR/dr),
+// with gR_p = g . T_p and s[e][k] = silu'(z_k) sum_b W1[b][k] dB_b/dr: the same GEMM as
+// R = h W2 on the same operand fragments, consumed where it leaves the accumulators (the
+// transpose GEMM of gR needs gR split per tile and a second copy of W2).  The gradient with
+// respect to the direction is a torque (aligned_gradient).  Both are summed over the quad's
+// channels, and the quad's share of the edge's position gradient,
+//   g_v = g_r u + (torque x u) / r,
+// goes to gv_part[quad][position].
 __global__ __launch_bounds__(64 * kMaceBwdWaves) __attribute__((amdgpu_waves_per_eu(3))) void mace_fused_backward_kernel(
     const float4* __restrict__ u4, const int* __restrict__ srcp, const int* __restrict__ dstp,
-    const v4u* __restrict__ h, const float* __restrict__ sg, const float* __restrict__ w2,
-    const float* __restrict__ x, const float* __restrict__ gout,
+    const v4u* __restrict__ h, const v4u* __restrict__ sg, const float* __restrict__ rl,
+    const float* __restrict__ w2, const float* __restrict__ x, const float* __restrict__ gout,
     const int64_t* __restrict__ wstart, float* __restrict__ gv_part, int64_t n_pos, int C,
     int n_quads, int ranges_per_xcd) {
     __shared__ v4u sW[kW2Frags * 64];
-    __shared__ v4u sV[kW2tFrags * 64];
     const MaceWg wg = mace_wg<kMaceBwdWaves>(n_quads, ranges_per_xcd);
     const int lane = threadIdx.x & 63, e16 = lane & 15, kk = lane >> 4;
     const int c0 = wg.quad * 4;
     mace_fill_w2(w2, C, c0, sW);
-    mace_fill_w2t(w2, C, c0, sV);
     __syncthreads();
     const int64_t p0 = wstart[wg.wave_range], p1 = wstart[wg.wave_range + 1];
     const int c = c0 + kk;
@@ -700,89 +508,61 @@ __global__ __launch_bounds__(64 * kMaceBwdWaves) __attribute__((amdgpu_waves_per
     const v4u* sA = sW + lane;
     float* gvq = gv_part + (int64_t)wg.quad * n_pos * 3;
     MaceTileIn cur;
-    if (p0 < p1) mace_load_tile(u4, srcp, dstp, h, min(p0 + e16, p1 - 1), kk, cur);
+    v4u sb[3 * kHSteps];
+    auto load_s = [&](int64_t pos) {
+        const v4u* sr = sg + pos * kHRow + kk;
+#pragma unroll
+        for (int j = 0; j < 3 * kHSteps; ++j) sb[j] = sr[4 * j];
+    };
+    if (p0 < p1) {
+        const int64_t pos = min(p0 + e16, p1 - 1);
+        mace_load_tile(u4, srcp, dstp, h, pos, kk, cur);
+        load_s(pos);
+    }
     for (int64_t t0 = p0; t0 < p1; t0 += 16) {
         const int64_t pos = t0 + e16;
         const bool valid = pos < p1;
-        const int64_t pc = valid ? pos : p1 - 1;
+        if (!valid) {
+#pragma unroll
+            for (int j = 0; j < 3 * kHSteps; ++j) cur.hb[j] = sb[j] = v4u{0, 0, 0, 0};
+        }
+        float rr[kNumPaths], ss[kNumPaths];
+        const v4u* const hp[2] = {cur.hb, sb};
+        float* const rp[2] = {rr, ss};
+        mace_tile_weights<2>(sA, hp, rp);
         float xs[16], g[16];
         load_row16(x + ((int64_t)cur.s * C + cc) * 16, xs);
         load_row16(gout + ((int64_t)cur.d * C + cc) * 16, g);
-        if (!valid) {
-#pragma unroll
-            for (int j = 0; j < 3 * kHSteps; ++j) cur.hb[j] = v4u{0, 0, 0, 0};
-        }
-        float rr[kNumPaths];
-        mace_tile_weights(sA, cur.hb, rr);
         if (!(valid && cok)) {
 #pragma unroll
             for (int o = 0; o < 16; ++o) g[o] = 0.0f;
         }
-        float Y[16];
-        sh_forward<3>(cur.u.x, cur.u.y, cur.u.z, Y);
-        // gY of the pair, and gR_p = g . T_p per path, every eight into the transpose GEMM
-        v4f gh[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) gh[j] = v4f{0.f, 0.f, 0.f, 0.f};
-        float gy[16], gR[8];
-        // (W2 read per tile through an opaque base, as in mace_tile_weights)
-        int wbase = 0;
-        asm volatile("" : "+v"(wbase));
-        const v4u* sVt = sV + lane + wbase;
-        mace_grad_y(xs, g, Y, rr, gy, [&](auto pp, float gr) {
-            constexpr int i = grad_slot(decltype(pp)::value), q = i / 8;
-            gR[i % 8] = gr;
-            if constexpr (i % 8 == 7 || i == kNumPaths - 1) {
-#pragma unroll
-                for (int z = i % 8 + 1; z < 8; ++z) gR[z] = 0.0f;
-                // (barriers: hoisted into the products, the fragments' reads spill)
-                __builtin_amdgcn_sched_barrier(0);
-                const Bf3 b = bf16_split8_finite(gR);
-                static_for<4>([&](auto jj) {
-                    constexpr int j = decltype(jj)::value;
-                    const v4u* f = sVt + (q * 4 + j) * 3 * 64;
-                    const Bf3 a{f[0], f[64], f[128]};
-                    mfma_bf16x6(a, b, gh[j], gh[j]);
-                    if constexpr (j % 2 == 1) __builtin_amdgcn_sched_barrier(0);
-                });
-            }
-        });
-        // the next tile's operands and this tile's s, in flight during the reductions
-        MaceTileIn nxt;
-        const int64_t t1 = t0 + 16;
-        mace_load_tile(u4, srcp, dstp, h, t1 < p1 ? min(t1 + e16, p1 - 1) : p1 - 1, kk, nxt);
-        const float4* sr = reinterpret_cast<const float4*>(sg + pc * kHidden + 4 * kk);
-        float4 sv[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sv[j] = sr[4 * j];
+        AlignedFrame f;
+        mace_frame(cur.u, rr, ss, f);
+        float tx, tz, gr;
+        aligned_gradient(f, xs, g, rr, ss, tx, tz, gr);
+        // the next tile's operands, in flight during the reductions
+        const float4 u = cur.u;
+        const int64_t t1 = t0 + 16, np = t1 < p1 ? min(t1 + e16, p1 - 1) : p1 - 1;
+        mace_load_tile(u4, srcp, dstp, h, np, kk, cur);
+        load_s(np);
         // summed over the quad's channels (rows of the wave)
-#pragma unroll
-        for (int b = 0; b < 16; ++b) {
-            gy[b] += __shfl_xor(gy[b], 16, 64);
-            gy[b] += __shfl_xor(gy[b], 32, 64);
-        }
-        float gux, guy, guz;
-        sh_backward<3>(cur.u.x, cur.u.y, cur.u.z, Y, gy, gux, guy, guz);
-        // g_r: D[k][e] of the lane's k = 16 j + 4 (lane / 16) + r against s[e][k]
-        float gr = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            gr = fmaf(gh[j][0], sv[j].x, gr);
-            gr = fmaf(gh[j][1], sv[j].y, gr);
-            gr = fmaf(gh[j][2], sv[j].z, gr);
-            gr = fmaf(gh[j][3], sv[j].w, gr);
-        }
+        tx += __shfl_xor(tx, 16, 64);
+        tz += __shfl_xor(tz, 16, 64);
         gr += __shfl_xor(gr, 16, 64);
+        tx += __shfl_xor(tx, 32, 64);
+        tz += __shfl_xor(tz, 32, 64);
         gr += __shfl_xor(gr, 32, 64);
         if (valid && kk == 0) {
-            const float ux = cur.u.x, uy = cur.u.y, uz = cur.u.z, ir = 1.0f / cur.u.w;
-            const float dot = ux * gux + uy * guy + uz * guz;
+            // in the aligned frame the unit vector moves by (-tz, 0, tx): back by the tilt and
+            // the turn
+            const float c = fminf(u.z, 1.0f), s = u.w, ir = 1.0f / rl[pos];
+            const float ax = -tz * ir, az = c * tx * ir;
             float* o = gvq + pos * 3;
-            o[0] = gr * ux + (gux - ux * dot) * ir;
-            o[1] = gr * uy + (guy - uy * dot) * ir;
-            o[2] = gr * uz + (guz - uz * dot) * ir;
+            o[0] = gr * s * u.y + fmaf(ax, u.x, az * u.y);
+            o[1] = gr * c - s * tx * ir;
+            o[2] = gr * s * u.x + fmaf(-ax, u.y, az * u.x);
         }
-        cur = nxt;
     }
 }
 
@@ -836,7 +616,7 @@ __global__ void mace_worker_starts_kernel(const int64_t* __restrict__ pos0, int6
     wstart[w] = min(pos0[lo], n_edges);
 }
 
-// Per position p (edge e = perm[p]): unit vector and length, source, destination,
+// Per position p (edge e = perm[p]): direction (and length), source, destination,
 // h = silu(B(r) W1 + b1); with sg, also s[k] = silu'(z_k) sum_b W1[b][k] dB_b/dr.
 // Sixteen lanes per position: lane q evaluates Bessel function q % 8 (one sincos)
 // and shares it with the position's other lanes, then forms hidden units
@@ -847,7 +627,7 @@ __global__ __launch_bounds__(256) void mace_prep_kernel(
     const int64_t* __restrict__ dst, const int64_t* __restrict__ perm,
     const float* __restrict__ w1, const float* __restrict__ b1, float rc, int64_t n_edges,
     float4* __restrict__ u4, int* __restrict__ srcp, int* __restrict__ dstp,
-    v4u* __restrict__ h, float* __restrict__ sg) {
+    v4u* __restrict__ h, v4u* __restrict__ sg, float* __restrict__ rl) {
     __shared__ float sW[kNBasis * kHidden + kHidden];
     for (int i = threadIdx.x; i < kNBasis * kHidden + kHidden; i += blockDim.x)
         sW[i] = i < kNBasis * kHidden ? w1[i] : b1[i - kNBasis * kHidden];
@@ -863,9 +643,14 @@ __global__ __launch_bounds__(256) void mace_prep_kernel(
     edge_vector(pos, s, d, bx.box, bx.inv, v);
     const float r = normalize3(v[0], v[1], v[2]);
     if (valid && q == 0) {
-        u4[p] = make_float4(v[0], v[1], v[2], r);
+        // direction (aligned.h): u = (s sin f, c, s cos f); along the axis any turn serves
+        const float s2 = sqrtf(v[0] * v[0] + v[2] * v[2]);
+        const float is = s2 > 0.0f ? 1.0f / s2 : 0.0f;
+        const bool none = r <= 1e-10f;  // (the length's lower bound)
+        u4[p] = make_float4(s2 > 0.0f ? v[2] * is : 1.0f, v[0] * is, none ? 2.0f : v[1], s2);
         srcp[p] = (int)s;
         dstp[p] = (int)d;
+        if (rl) rl[p] = r;
     }
     // Bessel function k = q % 8 of this position, with the envelope
     const float dd = r / rc;
@@ -907,16 +692,18 @@ __global__ __launch_bounds__(256) void mace_prep_kernel(
             sd[t] = sgm * (1.0f + acc * (1.0f - sgm)) * qq;
         }
     }
-    // h in three bf16 parts, [part][k] (hidden units 4q .. 4q + 3 of each part here)
-    const float z8[8] = {z[0], z[1], z[2], z[3], 0.f, 0.f, 0.f, 0.f};
-    const Bf3 zs = bf16_split8(z8);
-    if (valid) {
-        uint2* hr = reinterpret_cast<uint2*>(h + p * kHRow) + q;
-        hr[0] = make_uint2(zs.h[0], zs.h[1]);
-        hr[kHidden / 4] = make_uint2(zs.m[0], zs.m[1]);
-        hr[kHidden / 2] = make_uint2(zs.l[0], zs.l[1]);
-        if (sg) reinterpret_cast<float4*>(sg + p * kHidden)[q] = make_float4(sd[0], sd[1], sd[2], sd[3]);
-    }
+    // h and s in three bf16 parts, [part][k] (hidden units 4q .. 4q + 3 of each part here)
+    auto store = [&](v4u* row, const float* v) {
+        const float v8[8] = {v[0], v[1], v[2], v[3], 0.f, 0.f, 0.f, 0.f};
+        const Bf3 b = bf16_split8(v8);
+        if (!valid) return;
+        uint2* o = reinterpret_cast<uint2*>(row) + q;
+        o[0] = make_uint2(b.h[0], b.h[1]);
+        o[kHidden / 4] = make_uint2(b.m[0], b.m[1]);
+        o[kHidden / 2] = make_uint2(b.l[0], b.l[1]);
+    };
+    store(h + p * kHRow, z);
+    if (sg) store(sg + p * kHRow, sd);
 }
 
 // out rows of destinations without edges (the fused kernel writes the others)
@@ -962,8 +749,8 @@ struct MaceWs {
     int64_t *deg, *pos0, *perm, *wstart;
     float4* u4;
     int *srcp, *dstp;
-    v4u* h;
-    float *sg, *gv_part, *gv;
+    v4u *h, *sg;
+    float *rl, *gv_part, *gv;
     size_t bytes;
 };
 
@@ -990,7 +777,8 @@ static MaceWs mace_ws(void* base, int64_t N, int64_t E, int C, bool backward) {
     w.dstp = static_cast<int*>(take(sizeof(int) * e));
     w.h = static_cast<v4u*>(take(sizeof(v4u) * kHRow * e));
     if (backward) {
-        w.sg = static_cast<float*>(take(sizeof(float) * kHidden * e));
+        w.sg = static_cast<v4u*>(take(sizeof(v4u) * kHRow * e));
+        w.rl = static_cast<float*>(take(sizeof(float) * e));
         w.gv_part = static_cast<float*>(take(sizeof(float) * 3 * e * (size_t)mace_quads(C)));
         w.gv = static_cast<float*>(take(sizeof(float) * 3 * e));
     }
@@ -1072,7 +860,7 @@ static int mace_prepare(const float* positions, const MaceBox& bx, const float* 
         w.pos0, N, E, sh.n_workers, w.wstart);
     mace_prep_kernel<<<(unsigned)ceil_div(E, kPrepPositions), 256, 0, stream>>>(
         positions, bx, src, dst, w.perm, w1, b1, cutoff, E, w.u4, w.srcp, w.dstp, w.h,
-        backward ? w.sg : nullptr);
+        backward ? w.sg : nullptr, backward ? w.rl : nullptr);
     return (int)hipGetLastError();
 }
 
@@ -1173,7 +961,7 @@ extern "C" int batteries_mace_backward(const float* positions, const float* box,
                       cutoff, sh, w, true, stream);
     if (rc != BM_OK) return rc;
     mace_fused_backward_kernel<<<sh.grid, 64 * kMaceBwdWaves, 0, stream>>>(
-        w.u4, w.srcp, w.dstp, w.h, w.sg, w2, node_features, grad_out, w.wstart, w.gv_part,
+        w.u4, w.srcp, w.dstp, w.h, w.sg, w.rl, w2, node_features, grad_out, w.wstart, w.gv_part,
         N_edges, C, sh.n_quads, sh.ranges_per_xcd);
     mace_gv_reduce_kernel<<<(unsigned)ceil_div(N_edges, 256), 256, 0, stream>>>(
         w.gv_part, w.perm, N_edges, sh.n_quads, w.gv);

@@ -108,3 +108,51 @@ def test_mixing_kernel_infinities(bm, dev):
     assert torch.equal(out[:, 11, 0], -torch.sign(x[:, 7, 0] * y[:, 0]) * float("inf"))
     out[:, 11, 0] = 0.0
     assert torch.isfinite(out).all()
+
+
+def _cubic(n_side, spacing, tilt):
+    """A cubic lattice: edges along the axes (y is the harmonics' pole) and the diagonals;
+    tilt displaces every second atom in x, so that its edges lie tilt off the pole."""
+    k = torch.arange(n_side, dtype=torch.float32) * spacing
+    pos = torch.stack(torch.meshgrid(k, k, k, indexing="ij"), -1).reshape(-1, 3).contiguous()
+    pos[1::2, 0] += tilt
+    return pos, torch.diag(torch.full((3,), n_side * spacing))
+
+
+@pytest.mark.parametrize("tilt", [0.0, 1e-7, 1e-3])
+def test_layer_edges_along_the_pole(bm, dev, tilt):
+    import batmobile
+    pos, cell = _cubic(4, 3.0, tilt)
+    c = 6
+    graph = batmobile.Graph(pos.to(dev), cell, 5.0, c)
+    layer = batmobile.MACEInteraction(c, 5.0, device=dev, generator=gen(72))
+    x = torch.randn(pos.shape[0], c, 16, generator=gen(73))
+    go = torch.randn(pos.shape[0], c, 16, generator=gen(74))
+    p = pos.to(dev).requires_grad_(True)
+    out = layer(graph, p, x.to(dev))
+    (gp,) = torch.autograd.grad(out, p, go.to(dev))
+    want, gwant = om.layer_and_position_grad(
+        pos.numpy(), torch.diagonal(cell).numpy().astype(np.float64), x.numpy(),
+        graph.src.cpu().numpy(), graph.dst.cpu().numpy(), layer.W1.cpu().numpy(),
+        layer.b1.cpu().numpy(), layer.W2.cpu().numpy(), 5.0, go.numpy())
+    for got, ref in ((out.detach(), want), (gp, gwant)):
+        d = got.cpu().double().numpy() - ref
+        assert np.linalg.norm(d) <= 4e-6 * np.linalg.norm(ref)
+
+
+def test_layer_self_loops(bm, dev):
+    """An edge of no length: Y = (1, 0, ...), so only the paths with l2 = 0 act.  The basis is
+    taken at r = 1e-10, where the self loops' messages are large: compared per destination."""
+    import batmobile
+    pos, cell = periodic_box(60, 81)
+    c = 5
+    graph = batmobile.Graph(pos.to(dev), cell, 5.0, c, self_loops=True)
+    assert (graph.src == graph.dst).sum().item() == 60
+    layer = batmobile.MACEInteraction(c, 5.0, device=dev, generator=gen(82))
+    x = torch.randn(60, c, 16, generator=gen(83))
+    out = layer(graph, pos.to(dev), x.to(dev)).cpu().double()
+    box = torch.diagonal(cell).numpy().astype(np.float64)
+    t = [torch.as_tensor(a.cpu().numpy().astype(np.float64))
+         for a in (x, layer.W1, layer.b1, layer.W2)]
+    want = om.layer(pos.double(), box, t[0], graph.src.cpu(), graph.dst.cpu(), t[1], t[2], t[3], 5.0)
+    assert (out - want).norm() <= 4e-6 * want.norm()
