@@ -156,3 +156,29 @@ def test_layer_self_loops(bm, dev):
          for a in (x, layer.W1, layer.b1, layer.W2)]
     want = om.layer(pos.double(), box, t[0], graph.src.cpu(), graph.dst.cpu(), t[1], t[2], t[3], 5.0)
     assert (out - want).norm() <= 4e-6 * want.norm()
+
+
+# the kernels that calls without a workspace take: two row tiles a workgroup, one, 128
+# output channels, and past 128 with the rows staged and not
+@pytest.mark.parametrize("n,ci,co", [(50, 32, 64), (17, 40, 24), (33, 24, 100), (9, 16, 130),
+                                     (5, 8, 600)])
+def test_backward_without_workspace(bm, dev, n, ci, co):
+    import ctypes
+    import os
+    repo = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    lib = ctypes.CDLL(os.path.join(repo, "batmobile-evo_amd", "lib", "libbatmobile_hip.so"))
+    P = ctypes.c_void_p
+    fn = lib.batteries_tensor_product_backward_l3
+    fn.restype = ctypes.c_int
+    fn.argtypes = [P] * 7 + [ctypes.c_int64, ctypes.c_int, ctypes.c_int, P, ctypes.c_size_t, P]
+    x, y, w, g = (t.to(dev) for t in _product_inputs(n, ci, co, 91))
+    gx = torch.full_like(x, float("nan"))
+    gy = torch.full_like(y, float("nan"))
+    p = [P(t.data_ptr()) for t in (x, y, w, g, gx, gy)]
+    stream = P(torch.cuda.current_stream().cuda_stream)
+    assert fn(*p, None, n, ci, co, None, 0, stream) == 0
+    torch.cuda.synchronize()
+    wx, wy, _ = otp.tensor_product_backward(*(t.cpu().double().numpy() for t in (x, y, w, g)))
+    for got, ref in ((gx, wx), (gy, wy)):
+        d = got.cpu().double().numpy() - ref
+        assert np.linalg.norm(d) <= 1e-6 * np.linalg.norm(ref)
