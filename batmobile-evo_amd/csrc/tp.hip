@@ -792,6 +792,18 @@ constexpr int mix_unit_path(int k, int L, bool fwd) {
     return -1;
 }
 
+// The next entry of entry i's path with its (a, o), or -1 (there are at most two).
+constexpr int mix_next_of_pair(int i) {
+    for (int j = i + 1; j < kPathEntry[kCG[i].p + 1]; ++j)
+        if (kCG[j].a == kCG[i].a && kCG[j].o == kCG[i].o) return j;
+    return -1;
+}
+constexpr bool mix_pairs_at_most_two() {
+    for (int i = 0; i < kNumEntries; ++i)
+        if (mix_next_of_pair(i) >= 0 && mix_next_of_pair(mix_next_of_pair(i)) >= 0) return false;
+    return true;
+}
+static_assert(mix_pairs_at_most_two(), "an (a, o) of a path with more than two b");
 // Entry i is the first of its path with its (a, o).
 constexpr bool mix_first_of_pair(int i) {
     for (int j = kPathEntry[kCG[i].p]; j < i; ++j)
@@ -943,10 +955,8 @@ __device__ __forceinline__ void mix_unit(const float* __restrict__ xin, float* y
                         if constexpr ((FWD ? e.a : e.o) == z && mix_first_of_pair(i)) {
                             constexpr int ai = (FWD ? e.o : e.a) - A0;
                             float cy = e.c * yk[e.b];
-                            static_for<kPathEntry[p + 1] - 1 - i>([&](auto ff) {
-                                constexpr CGEntry f = kCG[i + 1 + decltype(ff)::value];
-                                if constexpr (f.a == e.a && f.o == e.o) cy = fmaf(f.c, yk[f.b], cy);
-                            });
+                            constexpr int j = mix_next_of_pair(i);
+                            if constexpr (j >= 0) cy = fmaf(kCG[j].c, yk[kCG[j].b], cy);
                             float sacc = 0.0f;
 #pragma unroll
                             for (int r = 0; r < 4; ++r) {
@@ -955,11 +965,7 @@ __device__ __forceinline__ void mix_unit(const float* __restrict__ xin, float* y
                             }
                             if constexpr (!FWD) {
                                 gyp[e.b] = fmaf(e.c, sacc, gyp[e.b]);
-                                static_for<kPathEntry[p + 1] - 1 - i>([&](auto ff) {
-                                    constexpr CGEntry f = kCG[i + 1 + decltype(ff)::value];
-                                    if constexpr (f.a == e.a && f.o == e.o)
-                                        gyp[f.b] = fmaf(f.c, sacc, gyp[f.b]);
-                                });
+                                if constexpr (j >= 0) gyp[kCG[j].b] = fmaf(kCG[j].c, sacc, gyp[kCG[j].b]);
                             }
                         }
                     });
