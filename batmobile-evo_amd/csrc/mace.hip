@@ -643,11 +643,21 @@ __global__ __launch_bounds__(256) void mace_prep_kernel(
     edge_vector(pos, s, d, bx.box, bx.inv, v);
     const float r = normalize3(v[0], v[1], v[2]);
     if (valid && q == 0) {
-        // direction (aligned.h): u = (s sin f, c, s cos f); along the axis any turn serves
-        const float s2 = sqrtf(v[0] * v[0] + v[2] * v[2]);
-        const float is = s2 > 0.0f ? 1.0f / s2 : 0.0f;
+        // direction (aligned.h): u = (s sin f, c, s cos f); along the axis any turn serves.
+        // The off-axis part is scaled before it is squared: below 1e-19 its square is
+        // subnormal, and (cos f, sin f) would not be of unit length.
+        const float m = fmaxf(fabsf(v[0]), fabsf(v[2]));
+        float cf = 1.0f, sf = 0.0f, s2 = fabsf(v[0] + v[2]);  // (0, or NaN)
+        if (m > 0.0f) {
+            sf = v[0] / m;
+            cf = v[2] / m;
+            const float h = sqrtf(cf * cf + sf * sf), ih = 1.0f / h;
+            sf *= ih;
+            cf *= ih;
+            s2 = m * h;
+        }
         const bool none = r <= 1e-10f;  // (the length's lower bound)
-        u4[p] = make_float4(s2 > 0.0f ? v[2] * is : 1.0f, v[0] * is, none ? 2.0f : v[1], s2);
+        u4[p] = make_float4(cf, sf, none ? 2.0f : v[1], s2);
         srcp[p] = (int)s;
         dstp[p] = (int)d;
         if (rl) rl[p] = r;

@@ -111,20 +111,27 @@ def test_mixing_kernel_infinities(bm, dev):
 
 
 def _cubic(n_side, spacing, tilt):
-    """A cubic lattice: edges along the axes (y is the harmonics' pole) and the diagonals;
-    tilt displaces every second atom in x, so that its edges lie tilt off the pole."""
+    """A cubic lattice: edges along the axes (y is the harmonics' pole) and the diagonals.
+    tilt displaces every second plane along y in x and (by 0.7 of it) in z, so that the y edges
+    of the atoms at x = 0 or z = 0, where a tilt of any size is kept, lie that far off the pole."""
     k = torch.arange(n_side, dtype=torch.float32) * spacing
-    pos = torch.stack(torch.meshgrid(k, k, k, indexing="ij"), -1).reshape(-1, 3).contiguous()
-    pos[1::2, 0] += tilt
-    return pos, torch.diag(torch.full((3,), n_side * spacing))
+    pos = torch.stack(torch.meshgrid(k, k, k, indexing="ij"), -1)
+    pos[:, 1::2, :, 0] += tilt
+    pos[:, 1::2, :, 2] += 0.7 * tilt
+    return pos.reshape(-1, 3).contiguous(), torch.diag(torch.full((3,), n_side * spacing))
 
 
-@pytest.mark.parametrize("tilt", [0.0, 1e-7, 1e-3])
+# 1e-22 to 1e-20: the square of the off-axis part of u is subnormal or 0; below, in reach of
+# rounding and not
+@pytest.mark.parametrize("tilt", [0.0, 4e-23, 1e-22, 1e-21, 1e-20, 1e-19, 1e-7, 1e-4, 1e-3])
 def test_layer_edges_along_the_pole(bm, dev, tilt):
     import batmobile
     pos, cell = _cubic(4, 3.0, tilt)
     c = 6
     graph = batmobile.Graph(pos.to(dev), cell, 5.0, c)
+    if tilt > 0.0:  # edges of the plane x = 0 keep the tilt
+        dx = (pos[graph.dst.cpu()] - pos[graph.src.cpu()])[:, 0].abs()
+        assert (dx == torch.tensor(tilt)).sum().item() >= 32
     layer = batmobile.MACEInteraction(c, 5.0, device=dev, generator=gen(72))
     x = torch.randn(pos.shape[0], c, 16, generator=gen(73))
     go = torch.randn(pos.shape[0], c, 16, generator=gen(74))
