@@ -335,25 +335,46 @@ __device__ __forceinline__ int dpp_next_i(int v) {  // lane e + 1 of the 16-lane
     return __builtin_amdgcn_update_dpp(0, v, 0x101, 0xF, 0xF, false);
 }
 
-// The frame of edge direction u = (cos f, sin f, c, s).  c = 2 marks an edge of no length:
-// its Y is (1, 0, ...), so only the paths with l2 = 0 act, which need no direction.
-__device__ __forceinline__ void mace_frame(const float4& u, float* r, float* s, AlignedFrame& f) {
-    const bool none = u.z > 1.5f;
-    if (__any(none)) {
+// The frame of edge direction u = (cos f, sin f, c, s); c and s are also returned.
+//
+// An edge shorter than the length's lower bound kMinLength has u = v / kMinLength, of length
+// rho < 1 (0 for a self loop), and Y_l(u) = rho^l Y_l(u / rho).  It is marked by a negative s
+// (-0 counts) and stored as rho (c, -s).  Its weights r are taken times rho^l2.  In the backward
+// (GRAD) the length is a constant there, so the gradient is that with respect to u alone, along
+// u / rho as well as across: with r times rho^(l2 - 1) (0 for l2 = 0, whose Y is a constant) the
+// torque is the part across times kMinLength, and s = l2 r / kMinLength gives the part along.
+constexpr float kMinLength = 1e-10f;
+template <bool GRAD>
+__device__ __forceinline__ void mace_frame(const float4& u, float* r, float* s, AlignedFrame& f,
+                                           float& c, float& sn) {
+    c = u.z;
+    sn = u.w;
+    const bool tiny = __float_as_int(u.w) < 0;
+    if (__any(tiny)) {
+        const float rho = tiny ? sqrtf(c * c + sn * sn) : 1.0f;
+        if (tiny) {
+            c = rho > 0.0f ? c / rho : 1.0f;
+            sn = rho > 0.0f ? -sn / rho : 0.0f;
+        }
+        const float pw[4] = {1.0f, rho, rho * rho, rho * rho * rho};
 #pragma unroll
-        for (int p = 0; p < kNumPaths; ++p)
-            if (kPathL[p][1] > 0) {
-                r[p] = none ? 0.0f : r[p];
-                s[p] = none ? 0.0f : s[p];
+        for (int p = 0; p < kNumPaths; ++p) {
+            const int l2 = kPathL[p][1];
+            if constexpr (GRAD) {
+                r[p] = l2 > 0 ? r[p] * pw[l2 > 0 ? l2 - 1 : 0] : (tiny ? 0.0f : r[p]);
+                s[p] = tiny ? (float)l2 * r[p] / kMinLength : s[p];
+            } else if (l2 > 0) {
+                r[p] *= pw[l2];
             }
+        }
     }
-    aligned_frame(u.x, u.y, none ? 1.0f : u.z, u.w, f);
+    aligned_frame(u.x, u.y, c, sn, f);
 }
 
 // One tile's per-position operands (pos clamped into the range by the caller).
 struct MaceTileIn {
     v4u hb[3 * kHSteps];
-    float4 u;  // direction (cos f, sin f, c, s)
+    float4 u;  // direction (mace_frame)
     int s, d;
 };
 
@@ -467,7 +488,8 @@ mace_fused_forward_kernel(const float4* __restrict__ u4, const int* __restrict__
         float xs[16];
         load_row16(x + ((int64_t)cur.s * C + cc) * 16, xs);
         AlignedFrame f;
-        mace_frame(cur.u, rr, rr, f);
+        float c1, s1;
+        mace_frame<false>(cur.u, rr, nullptr, f, c1, s1);
         float m[16];
         aligned_message(f, xs, rr, m);
         mace_stage_tile(m, e16, kk, sT);
@@ -538,11 +560,12 @@ __global__ __launch_bounds__(64 * kMaceBwdWaves) __attribute__((amdgpu_waves_per
             for (int o = 0; o < 16; ++o) g[o] = 0.0f;
         }
         AlignedFrame f;
-        mace_frame(cur.u, rr, ss, f);
+        float c1, s1;
+        mace_frame<true>(cur.u, rr, ss, f, c1, s1);
         float tx, tz, gr;
         aligned_gradient(f, xs, g, rr, ss, tx, tz, gr);
         // the next tile's operands, in flight during the reductions
-        const float4 u = cur.u;
+        const float cf = cur.u.x, sf = cur.u.y;
         const int64_t t1 = t0 + 16, np = t1 < p1 ? min(t1 + e16, p1 - 1) : p1 - 1;
         mace_load_tile(u4, srcp, dstp, h, np, kk, cur);
         load_s(np);
@@ -556,12 +579,12 @@ __global__ __launch_bounds__(64 * kMaceBwdWaves) __attribute__((amdgpu_waves_per
         if (valid && kk == 0) {
             // in the aligned frame the unit vector moves by (-tz, 0, tx): back by the tilt and
             // the turn
-            const float c = fminf(u.z, 1.0f), s = u.w, ir = 1.0f / rl[pos];
-            const float ax = -tz * ir, az = c * tx * ir;
+            const float ir = 1.0f / rl[pos];
+            const float ax = -tz * ir, az = c1 * tx * ir;
             float* o = gvq + pos * 3;
-            o[0] = gr * s * u.y + fmaf(ax, u.x, az * u.y);
-            o[1] = gr * c - s * tx * ir;
-            o[2] = gr * s * u.x + fmaf(-ax, u.y, az * u.x);
+            o[0] = gr * s1 * sf + fmaf(ax, cf, az * sf);
+            o[1] = gr * c1 - s1 * tx * ir;
+            o[2] = gr * s1 * cf + fmaf(-ax, sf, az * cf);
         }
     }
 }
@@ -656,8 +679,12 @@ __global__ __launch_bounds__(256) void mace_prep_kernel(
             cf *= ih;
             s2 = m * h;
         }
-        const bool none = r <= 1e-10f;  // (the length's lower bound)
-        u4[p] = make_float4(cf, sf, none ? 2.0f : v[1], s2);
+        float c = v[1];
+        if (r <= kMinLength) {  // (marked: mace_frame; also a NaN, which stays one)
+            if (s2 < 1e-15f && fabsf(c) < 1e-15f) c = s2 = 0.0f;  // (its square is subnormal)
+            s2 = copysignf(s2, -1.0f);
+        }
+        u4[p] = make_float4(cf, sf, c, s2);
         srcp[p] = (int)s;
         dstp[p] = (int)d;
         if (rl) rl[p] = r;

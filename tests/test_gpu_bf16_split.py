@@ -147,22 +147,62 @@ def test_layer_edges_along_the_pole(bm, dev, tilt):
         assert np.linalg.norm(d) <= 4e-6 * np.linalg.norm(ref)
 
 
+def _layer_against_oracle(dev, pos, cell, c, seed, **kw):
+    """(out, gpos, want, gwant) of a layer on the graph of pos."""
+    import batmobile
+    graph = batmobile.Graph(pos.to(dev), cell, 5.0, c, **kw)
+    layer = batmobile.MACEInteraction(c, 5.0, device=dev, generator=gen(seed))
+    n = pos.shape[0]
+    x = torch.randn(n, c, 16, generator=gen(seed + 1))
+    go = torch.randn(n, c, 16, generator=gen(seed + 2))
+    p = pos.to(dev).requires_grad_(True)
+    out = layer(graph, p, x.to(dev))
+    (gp,) = torch.autograd.grad(out, p, go.to(dev))
+    want, gwant = om.layer_and_position_grad(
+        pos.numpy(), torch.diagonal(cell).numpy().astype(np.float64), x.numpy(),
+        graph.src.cpu().numpy(), graph.dst.cpu().numpy(), layer.W1.cpu().numpy(),
+        layer.b1.cpu().numpy(), layer.W2.cpu().numpy(), 5.0, go.numpy())
+    return out.detach().cpu().double().numpy(), gp.cpu().double().numpy(), want, gwant
+
+
 def test_layer_self_loops(bm, dev):
     """An edge of no length: Y = (1, 0, ...), so only the paths with l2 = 0 act.  The basis is
-    taken at r = 1e-10, where the self loops' messages are large: compared per destination."""
-    import batmobile
+    taken at r = 1e-10.  Its position gradient cancels against that of its reverse, itself."""
     pos, cell = periodic_box(60, 81)
-    c = 5
-    graph = batmobile.Graph(pos.to(dev), cell, 5.0, c, self_loops=True)
-    assert (graph.src == graph.dst).sum().item() == 60
-    layer = batmobile.MACEInteraction(c, 5.0, device=dev, generator=gen(82))
-    x = torch.randn(60, c, 16, generator=gen(83))
-    out = layer(graph, pos.to(dev), x.to(dev)).cpu().double()
-    box = torch.diagonal(cell).numpy().astype(np.float64)
-    t = [torch.as_tensor(a.cpu().numpy().astype(np.float64))
-         for a in (x, layer.W1, layer.b1, layer.W2)]
-    want = om.layer(pos.double(), box, t[0], graph.src.cpu(), graph.dst.cpu(), t[1], t[2], t[3], 5.0)
-    assert (out - want).norm() <= 4e-6 * want.norm()
+    for got, ref in zip(*[iter(_layer_against_oracle(dev, pos, cell, 5, 82, self_loops=True)[i]
+                               for i in (0, 2, 1, 3))] * 2):
+        assert np.linalg.norm(got - ref) <= 4e-6 * np.linalg.norm(ref)
+
+
+# two atoms at one place, below the length's lower bound 1e-10 along the pole, across and
+# askew, below where squares are subnormal, and just above the bound
+@pytest.mark.parametrize("d", [(0.0, 0.0, 0.0), (0.0, 5e-11, 0.0), (5e-11, 0.0, 0.0),
+                               (3e-11, -4e-11, 6e-11), (2e-30, 1e-30, 0.0), (1e-10, 0.0, 1e-11)])
+def test_layer_short_edges(bm, dev, d):
+    """u = v / 1e-10 below the bound, the length a constant: the gradient of the two atoms is
+    of the order of 1e10, those of the others are as ever."""
+    pos = torch.tensor([[0.0, 0.0, 0.0], d, [1.0, 1.5, 2.0], [1.5, -1.0, 0.5]])
+    out, gp, want, gwant = _layer_against_oracle(dev, pos, torch.diag(torch.full((3,), 20.0)), 5, 72)
+    for got, ref in ((out, want), (gp[:2], gwant[:2]), (gp[2:], gwant[2:])):
+        assert np.linalg.norm(got - ref) <= 4e-6 * np.linalg.norm(ref)
+
+
+def test_layer_nan_position(bm, dev):
+    """A NaN coordinate reaches every component of the atom's neighbours."""
+    import batmobile
+    pos, cell = periodic_box(80, 91)
+    graph = batmobile.Graph(pos.to(dev), cell, 5.0, 4)
+    layer = batmobile.MACEInteraction(4, 5.0, device=dev, generator=gen(92))
+    x = torch.randn(80, 4, 16, generator=gen(93))
+    src, dst = graph.src.cpu(), graph.dst.cpu()
+    hit = torch.zeros(80, dtype=torch.bool)
+    hit[dst[src == 7]] = True
+    hit[7] = (dst == 7).any()
+    for k in range(3):
+        bad = pos.clone()
+        bad[7, k] = float("nan")
+        out = layer(graph, bad.to(dev), x.to(dev)).cpu()
+        assert torch.isnan(out[hit]).all() and torch.isfinite(out[~hit]).all()
 
 
 # the kernels that calls without a workspace take: two row tiles a workgroup, one, 128
