@@ -1403,6 +1403,12 @@ static bool mix_serves(int nk, int ni, const void* workspace, size_t bytes) {
     return workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
            (int64_t)kNumPaths * nk * ni * 4 <= INT32_MAX && bytes >= mix_packed_bytes(nk, ni);
 }
+// Rows per launch of the weighted forward and of the mixing kernel: keeps grid.x *
+// blockDim.x (at most 512 work-items per 16-row tile and group) below 2^32 - 1, the
+// dispatch limit, past which the grid wraps without an error; larger N runs as
+// consecutive launches over row ranges.
+constexpr int64_t kMaxRowsPerLaunch = int64_t(1) << 24;
+
 template <bool FWD>
 static int mix_launch(const float* z, const float* xin, const float* y, const float* w,
                       void* workspace, float* out, float* gy, int64_t n, int nk, int ni,
@@ -1411,18 +1417,27 @@ static int mix_launch(const float* z, const float* xin, const float* y, const fl
     const int total = kNumPaths * (int)(ceil_div(ni, 16) * ceil_div(nk, 32));
     tp_weighted_pack_kernel<FWD><<<(unsigned)ceil_div(total, kTpBlock / 64), kTpBlock, 0, stream>>>(
         w, wp, nk, ni, total);
-    const unsigned grid = (unsigned)ceil_div(n, kTile);
     // one channel tile has four units; LDS by the tiles of a pass
     const int tiles = std::min<int>(kMixTiles, (int)ceil_div(ni, 16));
     const int threads = 64 * (tiles == 1 ? 4 : kMixWaves);
     const size_t lds = (nk <= 32 ? 1 : 2) * (48u << 10) + tiles * (16u << 10);
-    if (nk <= 32)
-        tp_weighted_mix_kernel<FWD, 1><<<grid, threads, lds, stream>>>(z, xin, y, wp, out, gy, n,
-                                                                       nk, ni);
-    else
-        tp_weighted_mix_kernel<FWD, 2><<<grid, threads, lds, stream>>>(z, xin, y, wp, out, gy, n,
-                                                                       nk, ni);
-    return (int)hipGetLastError();
+    for (int64_t r0 = 0; r0 < n; r0 += kMaxRowsPerLaunch) {
+        const int64_t rows = std::min(kMaxRowsPerLaunch, n - r0);
+        const unsigned grid = (unsigned)ceil_div(rows, kTile);
+        const float* zr = z + r0 * nk * 16;
+        const float* xr = xin ? xin + r0 * ni * 16 : nullptr;
+        float* outr = out ? out + r0 * ni * 16 : nullptr;
+        float* gyr = gy ? gy + r0 * 16 : nullptr;
+        if (nk <= 32)
+            tp_weighted_mix_kernel<FWD, 1><<<grid, threads, lds, stream>>>(
+                zr, xr, y + r0 * 16, wp, outr, gyr, rows, nk, ni);
+        else
+            tp_weighted_mix_kernel<FWD, 2><<<grid, threads, lds, stream>>>(
+                zr, xr, y + r0 * 16, wp, outr, gyr, rows, nk, ni);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return (int)e;
+    }
+    return BM_OK;
 }
 
 // Row segments of the grad_W reduction: a fixed function of (N, C_in, C_out),
@@ -1488,11 +1503,6 @@ extern "C" int batteries_tensor_product_simple_backward_l3(const float* input1,
     return (int)hipGetLastError();
 }
 
-// Rows per launch of the weighted forward: keeps grid.x * blockDim.x (at most
-// 512 work-items per 16-row tile and group) below 2^32 - 1, the dispatch limit;
-// larger N runs as consecutive launches over row ranges.
-constexpr int64_t kFwdMaxRowsPerLaunch = int64_t(1) << 24;
-
 // Bytes that let batteries_tensor_product_l3_ws take the mixing kernel (0: it would not).
 extern "C" size_t batteries_tensor_product_l3_workspace_bytes(int64_t N, int C_in, int C_out) {
     if (C_in <= 0 || C_out <= 0 || !mix_forward_rows(N, C_in, C_out)) return 0;
@@ -1518,16 +1528,12 @@ extern "C" int batteries_tensor_product_l3_ws(const float* input1, const float* 
         return BM_ERR_ARG;
     const bool mix = mix_forward_rows(N, C_in, C_out) &&
                      mix_serves(C_in, C_out, workspace, workspace_bytes);
+    if (mix)
+        return mix_launch<true>(input1, nullptr, input2, weights, workspace, output, nullptr, N,
+                                C_in, C_out, stream);
     const int halves = C_in > 16 ? 2 : 1;  // input-channel chunks split over two wave halves
-    for (int64_t r0 = 0; r0 < N; r0 += kFwdMaxRowsPerLaunch) {
-        const int64_t rows = std::min(kFwdMaxRowsPerLaunch, N - r0);
-        if (mix) {
-            const int rc = mix_launch<true>(input1 + r0 * C_in * 16, nullptr, input2 + r0 * 16,
-                                            weights, workspace, output + r0 * C_out * 16, nullptr,
-                                            rows, C_in, C_out, stream);
-            if (rc != BM_OK) return rc;
-            continue;
-        }
+    for (int64_t r0 = 0; r0 < N; r0 += kMaxRowsPerLaunch) {
+        const int64_t rows = std::min(kMaxRowsPerLaunch, N - r0);
         const int64_t ntile = ceil_div(rows, kTile);
         // (row tile, group) pairs: tiles rounded up to 8, four groups each
         dim3 grid((unsigned)(ceil_div(ntile, 8) * 8 * kFwdGroups), (unsigned)ceil_div(C_out, 64), 1);

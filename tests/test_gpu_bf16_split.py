@@ -90,6 +90,23 @@ def test_mixing_kernel(bm, dev, n, ci, co):
         assert np.linalg.norm(got - ref) <= 1e-6 * np.linalg.norm(ref)
 
 
+def test_backward_past_the_grid_limit(bm, dev):
+    """More rows than one launch's work-items (2^32) hold: the last rows equal their own call's.
+    The inputs share one buffer (52 GB with the two gradients)."""
+    n, m = 2 ** 28 + 100, 1000
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("not enough free device memory")
+    y = torch.randn(n, 16, device=dev)
+    w = torch.randn(34, 1, 1, generator=gen(45)).to(dev)
+    x = y.view(n, 1, 16)
+    gx, gy, _ = bm.tensor_product_backward(x, y, w, x, True, True, False)
+    t = y[-m:].clone()
+    wx, wy, _ = bm.tensor_product_backward(t.view(m, 1, 16), t, w, t.view(m, 1, 16), True, True, False)
+    assert torch.equal(gx[-m:], wx) and torch.equal(gy[-m:], wy)
+    del x, y, gx, gy
+    torch.cuda.empty_cache()
+
+
 def test_mixing_kernel_infinities(bm, dev):
     """inf in component 0 of one row's channel reaches that row's outputs through the paths
     (0, l, l) only, as sign(W y) inf, and no other row; the same for an infinite weight."""
