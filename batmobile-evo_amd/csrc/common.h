@@ -110,22 +110,27 @@ __device__ __forceinline__ v4f mfma4(const float4 a, const float4 b, v4f acc) {
 //
 // fp32 MFMAs run at the vector FMA rate (2048 flops in 32 cycles per SIMD) and
 // share its issue with VALU work; v_mfma_f32_16x16x32_bf16 does 16,384 in 16.
-// An fp32 value is the exact sum of three bf16 values, x = h + m + l, each the
-// leading 8 bits of what is left (truncated, so the parts have the sign of x and
-// none overflows).  A product then is six bf16 products accumulated in fp32,
+// An fp32 value is the exact sum of three bf16 values, x = h + m + l: h is x and m what is
+// left of it, each rounded to nearest (8 significant bits), l the rest.  A product then is six
+// bf16 products accumulated in fp32,
 //   x y = hh' + (hm' + mh') + (hl' + mm' + lh'),
-// 2.7 times the fp32 MFMA rate; the dropped ml' + lm' are below 2^-23 of it.  With the
-// small products added while the accumulator is small (or in an accumulator of
-// their own) the error is below the fp32 MFMA chain's, which rounds after every
-// product: normal inputs, 2-norm relative, K = 64 / 512 / 4096: 0.78 / 1.4 / 4.0e-7
-// against 1.5 / 4.0 / 11e-7.  Parts below 2^-126 are flushed by the matrix cores:
-// values under 2^-110 lose their last bits.  Infinities: see bf16_split8.
+// 2.7 times the fp32 MFMA rate.  The dropped ml' + lm' are at most 2^-24 of it, 6e-9 (rms)
+// for normal inputs and of either sign, below fp32's own rounding (2^-24, 2.5e-8).  (Parts
+// truncated instead all have the sign of x: what is dropped is then a bias of up to 2^-21,
+// which sums of one sign keep.)  With the small products added while the accumulator is small
+// (or in an accumulator of their own) the error is below the fp32 MFMA chain's, which rounds
+// after every product: normal inputs, 2-norm relative, K = 64 / 512 / 4096: 0.49 / 1.3 /
+// 4.0e-7 against 1.4 / 4.0 / 12e-7.  The least bf16 is 2^-133 (subnormals are kept by the
+// conversion and by the matrix cores), so values under 2^-110 lose their last bits.
+// Infinities: see bf16_split8.
 //
 // v_mfma_f32_16x16x32_bf16: D (16x16) += A (16x32) * B (32x16).  Lane l supplies
 // A[l % 16][8 (l / 16) + j] and B[8 (l / 16) + j][l % 16] in element j, and holds
 // D[4 (l / 16) + r][l % 16] in element r (the accumulator layout of the fp32 form).
 // ---------------------------------------------------------------------------
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 // Eight fp32 values in three parts (the bits of a v8bf each).
@@ -138,57 +143,51 @@ __device__ __forceinline__ v4f mfma_bf16(v4u a, v4u b, v4f acc) {
                                                    __builtin_bit_cast(v8bf, b), acc, 0, 0, 0);
 }
 
-// (hi 16 bits of b, hi 16 bits of a) as two packed bf16
-__device__ __forceinline__ unsigned bf16_pack_hi(float a, float b) {
-    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+// a and b as two packed bf16, rounded to nearest (one v_cvt_pk_bf16_f32), and back
+__device__ __forceinline__ unsigned bf16_pack(float a, float b) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector((v2f{a, b}), v2bf));
 }
-__device__ __forceinline__ float bf16_trunc(float x) {
-    return __uint_as_float(__float_as_uint(x) & 0xffff0000u);
-}
+__device__ __forceinline__ float bf16_lo(unsigned p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float bf16_hi(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
 
-// The three parts of x[0..7], for finite x (an infinity leaves inf - inf = NaN in the
-// lower parts; a NaN stays a NaN in some part).
-__device__ __forceinline__ Bf3 bf16_split8_finite(const float* x) {
-    Bf3 s;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float a = x[2 * i], b = x[2 * i + 1];
-        const float ra = a - bf16_trunc(a), rb = b - bf16_trunc(b);
-        const float la = ra - bf16_trunc(ra), lb = rb - bf16_trunc(rb);
-        s.h[i] = bf16_pack_hi(a, b);
-        s.m[i] = bf16_pack_hi(ra, rb);
-        s.l[i] = bf16_pack_hi(la, lb);
-    }
-    return s;
-}
-// The same for any x: an infinity, with one in the wave, goes to the l part alone
-// (h = m = 0), which meets only the other factor's h part, so inf * y = +-inf (and
-// inf * 0 = NaN) as in fp32.
+// The three parts of x[0..7].  Values that bf16 rounds to infinity (from kBf16Max on) take
+// their leading bits as h instead; an infinity goes to the l part alone (h = m = 0), which
+// meets only the other factor's h part, so inf * y = +-inf (and inf * 0 = NaN) as in fp32.  A
+// NaN stays one in h.
+constexpr float kBf16Max = 0x1.ffp127f;
 __device__ __forceinline__ Bf3 bf16_split8(const float* x) {
+    Bf3 s;
     float mx = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(x[i]));
-    if (__builtin_expect(__any(mx == __builtin_inff()), 0)) {
-        Bf3 s;
+    if (__builtin_expect(__any(mx >= kBf16Max), 0)) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            float h[2], r[2], m[2], l[2];
+            float h[2], m[2], l[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const float v = x[2 * i + j];
-                const bool inf = fabsf(v) == __builtin_inff();
-                h[j] = inf ? 0.0f : bf16_trunc(v);
-                r[j] = v - h[j];
-                m[j] = inf ? 0.0f : bf16_trunc(r[j]);
-                l[j] = r[j] - m[j];
+                const bool inf = fabsf(v) == __builtin_inff(), big = fabsf(v) >= kBf16Max;
+                h[j] = inf ? 0.0f : (big ? bf16_hi(__float_as_uint(v)) : bf16_lo(bf16_pack(v, 0.0f)));
+                const float r = v - h[j];
+                m[j] = inf ? 0.0f : bf16_lo(bf16_pack(r, 0.0f));
+                l[j] = r - m[j];
             }
-            s.h[i] = bf16_pack_hi(h[0], h[1]);
-            s.m[i] = bf16_pack_hi(m[0], m[1]);
-            s.l[i] = bf16_pack_hi(l[0], l[1]);
+            s.h[i] = bf16_pack(h[0], h[1]);
+            s.m[i] = bf16_pack(m[0], m[1]);
+            s.l[i] = bf16_pack(l[0], l[1]);
         }
         return s;
     }
-    return bf16_split8_finite(x);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a = x[2 * i], b = x[2 * i + 1];
+        s.h[i] = bf16_pack(a, b);
+        const float ra = a - bf16_lo(s.h[i]), rb = b - bf16_hi(s.h[i]);
+        s.m[i] = bf16_pack(ra, rb);
+        s.l[i] = bf16_pack(ra - bf16_lo(s.m[i]), rb - bf16_hi(s.m[i]));
+    }
+    return s;
 }
 
 // acc += A B over one K = 32 step, the five small products into lo

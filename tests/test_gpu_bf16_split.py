@@ -90,6 +90,47 @@ def test_mixing_kernel(bm, dev, n, ci, co):
         assert np.linalg.norm(got - ref) <= 1e-6 * np.linalg.norm(ref)
 
 
+# Sums of few products, where the parts' own error shows: y = (1, 0, ...) leaves one path per
+# degree, so out and grad_input1 are sums of k products.  The dropped products are at most
+# 2^-24 of each and fp32 rounds a few times by at most 2^-24 (6e-8), by 2.5e-8 (rms); grad_input2
+# sums over channels and components besides.  same: one sign, and the leading bits at which
+# truncated parts would drop most.
+@pytest.mark.parametrize("same", [False, True])
+@pytest.mark.parametrize("k", [1, 4, 8])
+def test_short_sums_against_float64(bm, dev, k, same):
+    x, _, w, g = _product_inputs(3072, k, k, 47)
+    y = torch.zeros(3072, 16)
+    y[:, 0] = 1.0
+    if same:
+        v = 1.0 + 2.0 ** -7 - 2.0 ** -23
+        x, w, g = (torch.full_like(t, v) for t in (x, w, g))
+    out = bm.tensor_product(x.to(dev), y.to(dev), w.to(dev))
+    gx, gy, _ = bm.tensor_product_backward(x.to(dev), y.to(dev), w.to(dev), g.to(dev))
+    d = [t.double().numpy() for t in (x, y, w, g)]
+    wx, wy, _ = otp.tensor_product_backward(*d)
+    for got, ref, tol in ((out, otp.tensor_product(*d[:3]), 1e-7), (gx, wx, 1e-7), (gy, wy, 2e-7)):
+        assert np.linalg.norm(got.cpu().double().numpy() - ref) <= tol * np.linalg.norm(ref)
+
+
+def test_values_that_bf16_rounds_to_infinity(bm, dev):
+    """Up to the largest finite fp32 value: its products are those of fp32."""
+    n, c = 3072, 20
+    x, _, w, _ = _product_inputs(n, c, c, 48)
+    y = torch.zeros(n, 16)
+    y[:, 0] = 1.0
+    big = torch.tensor([3.4028234e38, -3.4e38, 3.3961775e38])  # (the last: the least such value)
+    x[5] = 0.0
+    x[5, :3, 0] = big
+    w[0, :3] = 0.25 * torch.eye(3, c)
+    w[0, 3:] = 0.0
+    out = bm.tensor_product(x.to(dev), y.to(dev), w.to(dev)).cpu()
+    assert torch.equal(out[5, :3, 0], 0.25 * big)
+    keep = [i for i in range(16) if i != 5]  # rows of the same wave
+    d = [t[keep].double().numpy() for t in (x, y)]
+    ref = otp.tensor_product(*d, w.double().numpy())
+    assert np.linalg.norm(out[keep].double().numpy() - ref) <= 1e-6 * np.linalg.norm(ref)
+
+
 def test_backward_past_the_grid_limit(bm, dev):
     """More rows than one launch's work-items (2^32) hold: the last rows equal their own call's.
     The inputs share one buffer (52 GB with the two gradients)."""
