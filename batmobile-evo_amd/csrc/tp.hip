@@ -836,15 +836,21 @@ __device__ __forceinline__ int mix_so(int row, int i, int c) {
 }
 
 // Weights split beforehand, [path][tile of i][32-channel step][part][lane] (1 KB each, zeros
-// past the channels).  One wave per (path, tile, step).
+// past the channels).  An odd number of steps from 3 on leaves the last chunk of 64 channels
+// one step: a zero fragment behind the path's tiles serves as the other (Z is zero there, and
+// an infinite weight would meet it as inf * 0).  One wave per fragment triple.
+__host__ __device__ constexpr int mix_steps(int nk) { return (nk + 31) / 32; }
+__host__ __device__ constexpr int mix_path_frags(int nk, int ni) {
+    return (ni + 15) / 16 * mix_steps(nk) + (mix_steps(nk) > 1 && mix_steps(nk) % 2 == 1 ? 1 : 0);
+}
 template <bool FWD>
 __global__ __launch_bounds__(kTpBlock) void tp_weighted_pack_kernel(const float* __restrict__ w,
                                                                     v4u* __restrict__ wp, int nk,
                                                                     int ni, int total) {
     const int id = blockIdx.x * (kTpBlock / 64) + (threadIdx.x >> 6);
     if (id >= total) return;  // uniform over the wave
-    const int lane = threadIdx.x & 63, nks = (nk + 31) / 32, nit = (ni + 15) / 16;
-    const int s = id % nks, it = id / nks % nit, p = id / (nks * nit);
+    const int lane = threadIdx.x & 63, nks = mix_steps(nk), npf = mix_path_frags(nk, ni);
+    const int p = id / npf, s = id % npf % nks, it = id % npf / nks;  // (zero fragment: past ni)
     const int i = it * 16 + (lane & 15), k = 32 * s + 8 * (lane >> 4);
     float v[8];
 #pragma unroll
@@ -861,8 +867,8 @@ __global__ __launch_bounds__(kTpBlock) void tp_weighted_pack_kernel(const float*
 }
 
 // One unit over the chunk of Z in sZ: wu = the fragments of path 0 for the unit's tile and
-// chunk, pstep = distance between paths, s1 = of the second step (0: there is
-// none, and Z is zero there).  sO holds the chunks' sums so far (first: the backward's x).
+// chunk, pstep = distance between paths, s1 = of the second step (or of the zero fragment).
+// sO holds the chunks' sums so far (first: the backward's x).
 template <bool FWD, int KS, int L>
 __device__ __forceinline__ void mix_unit(const float* __restrict__ xin, float* yb,
                                          const v4u* __restrict__ wu, int64_t pstep, int s1,
@@ -1009,8 +1015,8 @@ __global__ __launch_bounds__(64 * kMixWaves) void tp_weighted_mix_kernel(
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t row0 = (int64_t)blockIdx.x * kTile;
     const int rows = (int)min<int64_t>(kTile, n - row0);
-    const int nct = (ni + 15) / 16, nks = (nk + 31) / 32;
-    const int64_t pstep = (int64_t)nct * nks * 192, row_c = row0 + min(i16, rows - 1);
+    const int nct = (ni + 15) / 16, nks = mix_steps(nk);
+    const int64_t pstep = (int64_t)mix_path_frags(nk, ni) * 192, row_c = row0 + min(i16, rows - 1);
     float yb[16], gyp[16];
     load16(y, row_c * 16, yb);  // rows >= n reach discarded outputs
 #pragma unroll
@@ -1076,13 +1082,14 @@ __global__ __launch_bounds__(64 * kMixWaves) void tp_weighted_mix_kernel(
                     }
                 }
             __syncthreads();
-            const int s1 = KS > 1 && k0 / 32 + 1 < nks ? 192 : 0;
 #pragma clang loop unroll(disable)
             for (int u = 0; u < 2; ++u) {
                 const int unit = mix_unit_of(nt, wv, u);
                 if (unit < 0) continue;
                 const int it = unit >> 2, ct = c0 + it;
-                const v4u* wu = wp + ((int64_t)ct * nks + k0 / 32) * 192;
+                const int f0 = ct * nks + k0 / 32;
+                const v4u* wu = wp + (int64_t)f0 * 192;
+                const int s1 = k0 / 32 + 1 < nks ? 192 : (nct * nks - f0) * 192;
                 switch (unit & 3) {
                     case 0: mix_unit<FWD, KS, 0>(xin, yb, wu, pstep, s1, k0 == 0, ct, it, ni, row_c, sZ, sO, gyp); break;
                     case 1: mix_unit<FWD, KS, 1>(xin, yb, wu, pstep, s1, k0 == 0, ct, it, ni, row_c, sZ, sO, gyp); break;
@@ -1397,7 +1404,7 @@ static bool mix_forward_rows(int64_t n, int cin, int cout) {
     return n >= (cout > 8 * cin ? kMixRowsWide : kMixRows);
 }
 static size_t mix_packed_bytes(int nk, int ni) {
-    return (size_t)kNumPaths * ceil_div(ni, 16) * ceil_div(nk, 32) * 192 * sizeof(v4u);
+    return (size_t)kNumPaths * mix_path_frags(nk, ni) * 192 * sizeof(v4u);
 }
 static bool mix_serves(int nk, int ni, const void* workspace, size_t bytes) {
     return workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 &&
@@ -1414,7 +1421,7 @@ static int mix_launch(const float* z, const float* xin, const float* y, const fl
                       void* workspace, float* out, float* gy, int64_t n, int nk, int ni,
                       hipStream_t stream) {
     v4u* wp = static_cast<v4u*>(workspace);
-    const int total = kNumPaths * (int)(ceil_div(ni, 16) * ceil_div(nk, 32));
+    const int total = kNumPaths * mix_path_frags(nk, ni);
     tp_weighted_pack_kernel<FWD><<<(unsigned)ceil_div(total, kTpBlock / 64), kTpBlock, 0, stream>>>(
         w, wp, nk, ni, total);
     // one channel tile has four units; LDS by the tiles of a pass

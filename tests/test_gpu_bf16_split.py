@@ -168,6 +168,30 @@ def test_mixing_kernel_infinities(bm, dev):
     assert torch.isfinite(out).all()
 
 
+@pytest.mark.parametrize("nk", [65, 72, 96, 130])
+def test_mixing_kernel_infinite_weight_of_an_odd_step(bm, dev, nk):
+    """A last chunk of 1 to 32 contracted channels has no second step: an infinite weight in
+    its first one reaches one output channel, as sign(x y) inf or sign(g y) inf."""
+    n, i = 3072, 20
+    k = nk - 1
+    x, y, w, _ = _product_inputs(n, nk, i, 63)
+    w[0, k, 11] = float("inf")
+    out = bm.tensor_product(x.to(dev), y.to(dev), w.to(dev)).cpu()
+    assert torch.equal(out[:, 11, 0], torch.sign(x[:, k, 0] * y[:, 0]) * float("inf"))
+    out[:, 11, 0] = 0.0
+    assert torch.isfinite(out).all()
+    x, y, w, g = _product_inputs(100, i, nk, 64)
+    w[0, 11, k] = float("inf")
+    gx, gy, _ = bm.tensor_product_backward(x.to(dev), y.to(dev), w.to(dev), g.to(dev), True, True,
+                                           False)
+    gx, gy = gx.cpu(), gy.cpu()
+    assert torch.equal(gx[:, 11, 0], torch.sign(g[:, k, 0] * y[:, 0]) * float("inf"))
+    gx[:, 11, 0] = 0.0
+    assert torch.isfinite(gx).all()
+    assert torch.equal(gy[:, 0], torch.sign(x[:, 11, 0] * g[:, k, 0]) * float("inf"))
+    assert torch.isfinite(gy[:, 1:]).all()
+
+
 def _cubic(n_side, spacing, tilt):
     """A cubic lattice: edges along the axes (y is the harmonics' pole) and the diagonals.
     tilt displaces every second plane along y in x and (by 0.7 of it) in z, so that the y edges
