@@ -1392,16 +1392,35 @@ static int64_t bwd_xy_pairs(int64_t tiles) {
     return ceil_div(tiles, 2);
 }
 
-// The mixing kernel serves a call when the caller's workspace has room for the split
-// weights.  Forward: from kMixRows rows on; below, the weights' split and workgroups of 16
-// rows x all output channels (fewer than the compute units) cost more than they save (32 ->
-// 64 channels: 20.1 -> 23.5 us at 1,400 rows, 29.6 -> 24.4 at 3,072).  With many more output
-// than input channels the CG terms, here per output channel, weigh more: 8 -> 128 channels
-// 37.8 -> 40.8 us at 3,072 rows, 115 -> 111 at 10,000.  Backward: always (32 -> 64 channels
-// 35.9 -> 25.4 us at 100 rows, 462 -> 419 at 60,000; 48 -> 72: 1921 -> 876).
-constexpr int64_t kMixRows = 3072, kMixRowsWide = 8192;
+// The mixing kernel serves a call that its rule gives it and whose workspace has room for
+// the split weights.
+//
+// Forward: from kMixRows rows on; below, the weights' split and workgroups of 16 rows x all
+// output channels (fewer than the compute units) cost more than they save (32 -> 64 channels:
+// 20.1 -> 23.5 us at 1,400 rows, 29.6 -> 24.4 at 3,072).  With up to 16 input channels the fp32
+// kernel forms few products: its time goes as the rounds of 1,024 rows (four workgroups per
+// 16-row tile) and the 64-channel blocks of C_out, the mixing kernel's as the rounds of 4,096
+// rows (one workgroup per tile and compute unit) and the 16-channel tiles.  The latter serves
+// where it takes a round for 2.5 or fewer of the former's, 3.25 where C_out fills its blocks.
+// us, fp32 / mixing: 16 -> 64 channels 20.5 / 23.2 at 3,072 rows, 25.3 / 23.3 at 3,400, 29.6 /
+// 39.9 at 4,100, 37.3 / 41.3 at 5,400, 43.2 / 41.8 at 6,500, 51.5 / 60.1 at 8,200, 60.3 / 59.7 at
+// 10,000; 16 -> 112 51.5 / 64.1 at 4,100, 58.7 / 65.3 at 4,800, 75.6 / 65.6 at 6,500.  Up to 32
+// output channels two workgroups share a compute unit and it is always ahead.
+//
+// Backward: always (32 -> 64 channels 35.9 -> 25.4 us at 100 rows, 462 -> 419 at 60,000; 48 ->
+// 72: 1921 -> 876), but for many rows of one tile of input channels and two steps of output
+// channels, whose 112 KB leave a compute unit one workgroup of four waves: 16 -> 64 channels
+// 24.7 / 23.6 us at 1,000 rows, 26.5 / 28.8 at 3,500, 301 / 354 at 60,000; 16 -> 48 26.2 / 24.8 at
+// 4,000, 37.8 / 42.5 at 4,100.
+constexpr int64_t kMixRows = 3072, kMixRound = 4096, kFp32Round = 1024;
 static bool mix_forward_rows(int64_t n, int cin, int cout) {
-    return n >= (cout > 8 * cin ? kMixRowsWide : kMixRows);
+    if (n < kMixRows) return false;
+    const int64_t tiles = ceil_div(cout, 16);
+    if (cin > 16 || tiles <= 2) return true;
+    return 4 * ceil_div(n, kFp32Round) > (tiles % 4 == 0 ? 13 : 10) * ceil_div(n, kMixRound);
+}
+static bool mix_backward_rows(int64_t n, int cin, int cout) {
+    return cin > 16 || cout <= 32 || cout > 64 || n <= (cout <= 48 ? 4096 : 2560);
 }
 static size_t mix_packed_bytes(int nk, int ni) {
     return (size_t)kNumPaths * mix_path_frags(nk, ni) * 192 * sizeof(v4u);
@@ -1570,7 +1589,7 @@ extern "C" size_t batteries_tensor_product_backward_l3_workspace_bytes(int64_t N
     if (N <= 0 || C_in <= 0 || C_out <= 0) return 0;
     const size_t gw =
         with_weights ? batteries_tensor_product_backward_workspace_bytes(N, C_in, C_out) : 0;
-    return std::max(gw, mix_packed_bytes(C_out, C_in));
+    return mix_backward_rows(N, C_in, C_out) ? std::max(gw, mix_packed_bytes(C_out, C_in)) : gw;
 }
 
 // The weighted backward on a given workspace (null or `bytes` bytes; at least
@@ -1582,7 +1601,7 @@ static int tp_backward_run(const float* input1, const float* input2, const float
                            size_t bytes, hipStream_t stream) {
     float* gw_part = static_cast<float*>(workspace);
     if (grad_input1 || grad_input2) {
-        if (mix_serves(C_out, C_in, workspace, bytes)) {
+        if (mix_backward_rows(N, C_in, C_out) && mix_serves(C_out, C_in, workspace, bytes)) {
             const int rc = mix_launch<false>(grad_output, input1, input2, weights, workspace,
                                              grad_input1, grad_input2, N, C_out, C_in, stream);
             if (rc != BM_OK) return rc;

@@ -69,10 +69,11 @@ def _product_inputs(n, ci, co, seed):
 
 # rows: one below and at the forward's line, a last tile of 15 rows, single rows; channels:
 # parts of a tile, 1 to 4 tiles of a pass and past it, contracted channels of one 32-step, two,
-# a partial second, and past one chunk of 64
+# a partial second, and past one chunk of 64; the lines that the rounds of workgroups draw
 @pytest.mark.parametrize("n,ci,co", [(3071, 8, 8), (3072, 1, 3), (3087, 33, 17), (3073, 64, 65),
                                      (3072, 20, 130), (3088, 130, 20), (3072, 72, 48), (1, 40, 96),
-                                     (17, 48, 150), (8200, 4, 40)])
+                                     (17, 48, 150), (8200, 4, 40), (3072, 8, 64), (3073, 8, 64),
+                                     (4097, 12, 33), (5121, 16, 96), (2561, 16, 64)])
 def test_mixing_kernel(bm, dev, n, ci, co):
     x, y, w, g = _product_inputs(n, ci, co, 51)
     out = bm.tensor_product(x.to(dev), y.to(dev), w.to(dev)).cpu().double().numpy()
