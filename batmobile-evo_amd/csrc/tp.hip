@@ -1757,7 +1757,9 @@ extern "C" int batteries_tensor_product_backward_l3_noalloc(
         const int e = scratch_address(&part);
         if (e != BM_OK) return e;
     }
-    return tp_backward_run(input1, input2, weights, grad_output, grad_input1, grad_input2,
-                           grad_weights, N, C_in, C_out, part,
-                           part ? BATMOBILE_HIP_NOALLOC_SCRATCH_BYTES : 0, stream);
+    // the room of the workspace form's least workspace, not the whole array: the room decides
+    // which kernel forms grad_input1 and grad_input2, and both forms give the same bits
+    return tp_backward_run(
+        input1, input2, weights, grad_output, grad_input1, grad_input2, grad_weights, N, C_in, C_out,
+        part, part ? batteries_tensor_product_backward_workspace_bytes(N, C_in, C_out) : 0, stream);
 }

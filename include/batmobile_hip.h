@@ -103,7 +103,8 @@ int batteries_tensor_product_l3_ws(const float* input1, const float* input2, con
 
 /* Least workspace for batteries_tensor_product_backward_l3 with grad_weights != NULL (none is
  * needed without), and the workspace with which it is fastest (with_weights: grad_weights is
- * wanted). */
+ * wanted).  grad_input1 and grad_input2 agree to rounding between workspace sizes: with room
+ * for the split weights they come from the kernel that needs them. */
 size_t batteries_tensor_product_backward_l3_workspace_bytes(int64_t N, int C_in, int C_out,
                                                             int with_weights);
 size_t batteries_tensor_product_backward_workspace_bytes(int64_t N, int C_in, int C_out);
@@ -124,8 +125,9 @@ int batteries_tensor_product_backward_l3(const float* input1, const float* input
 /* The backward above without any allocation, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  No counterpart in the reference.  Same arguments and results
- * as batteries_tensor_product_backward_l3 minus the workspace: the grad_W partials
- * live in a static device array of BATMOBILE_HIP_NOALLOC_SCRATCH_BYTES per GPU.
+ * as batteries_tensor_product_backward_l3 with its least workspace (none without
+ * grad_weights), bit for bit: the workspace lives in a static device array of
+ * BATMOBILE_HIP_NOALLOC_SCRATCH_BYTES per GPU.
  * Returns BATMOBILE_HIP_ERR_SCRATCH (and touches nothing) when grad_weights is
  * requested and batteries_tensor_product_backward_workspace_bytes(N, C_in, C_out)
  * exceeds it.  The partials fit for every N when 3 ceil(C_in/16) ceil(C_out/64)

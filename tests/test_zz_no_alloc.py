@@ -89,6 +89,27 @@ def test_noalloc_backward_equals_workspace_backward(dev):
         assert normwise_err(got[1][:k].cpu(), wy) <= 1e-4
 
 
+# shapes whose split weights take more room than the grad_W partials, and less
+@pytest.mark.parametrize("n,cin,cout", [(50, 8, 8), (3, 40, 70), (900, 16, 40), (4000, 24, 24)])
+def test_noalloc_backward_takes_the_workspace_forms_kernels(dev, n, cin, cout):
+    lib = _lib()
+    x, y, w, g = _inputs(n, cin, cout, 531, dev)
+    for a, b in zip(_run(lib, False, x, y, w, g, dev), _run(lib, True, x, y, w, g, dev)):
+        assert torch.equal(a, b)
+    # without grad_weights: the workspace form without a workspace
+    res = []
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for form in range(2):
+        gx, gy = torch.full_like(x, float("nan")), torch.full_like(y, float("nan"))
+        args = [_ptr(x), _ptr(y), _ptr(w), _ptr(g), _ptr(gx), _ptr(gy), None, n, cin, cout]
+        rc = (lib.batteries_tensor_product_backward_l3_noalloc(*args, stream) if form else
+              lib.batteries_tensor_product_backward_l3(*args, None, 0, stream))
+        torch.cuda.synchronize()
+        assert rc == 0
+        res.append((gx, gy))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+
+
 def test_noalloc_backward_weight_grad_against_oracle(dev):
     lib = _lib()
     n, cin, cout = 300, 8, 16
