@@ -851,17 +851,21 @@ static int mace_cu_count() {
 
 // Launch shape of a fused kernel: every quad of a position range on one XCD.  The
 // workgroups of an XCD, ranges x quads, run in rounds of its resident ones (occupancy
-// from the runtime for this kernel); a range is a 1 / ranges share of the work, so the
-// time goes as rounds / ranges.  The ranges are the fewest that bring it within 5% of
-// the least over the first eight counts from one full round on: at C = 80 (20 quads on
-// 32 slots) one range leaves 12 slots idle, three fill 60 of 64.
+// from the runtime for this kernel).  A round fills the workgroup's W2 fragments, which
+// takes about as long as a tile of each wave (7 to 8 us), and then the wave's share of the
+// tiles, so the time goes as rounds (1 + tiles / waves).  The ranges are the fewest that
+// bring it within 5% of the least over the first eight counts from one full round on.
+// C = 80 (20 quads on 32 slots): one range leaves 12 slots idle, three fill 60 of 64, from
+// 7,600 edges on.  C = 112 (28 quads): eight ranges fill seven rounds; by rounds / ranges
+// alone they were taken at any size, us forward with them / now at 60, 1,000 and 4,000
+// atoms of 30 edges: 92 / 48, 170 / 139, 425 / 401.
 struct MaceShape {
     int n_quads, ranges_per_xcd, n_workers;
     unsigned grid;
 };
 
 template <typename K>
-static int mace_shape(K kernel, int waves, int C, MaceShape* sh) {
+static int mace_shape(K kernel, int waves, int C, int64_t n_edges, MaceShape* sh) {
     int occ = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, 64 * waves, 0) != hipSuccess ||
         occ < 1)
@@ -870,7 +874,10 @@ static int mace_shape(K kernel, int waves, int C, MaceShape* sh) {
     sh->n_quads = mace_quads(C);
     const int slots = per_xcd * occ, first = std::max(1, slots / sh->n_quads);
     const int last = std::min(first + 7, kMaceMaxWorkers / (8 * waves));
-    auto cost = [&](int r) { return (double)ceil_div((int64_t)r * sh->n_quads, slots) / r; };
+    const double tiles = (double)ceil_div(n_edges, 16);
+    auto cost = [&](int r) {
+        return ceil_div((int64_t)r * sh->n_quads, slots) * (1.0 + tiles / (8.0 * r * waves));
+    };
     int best = first;
     for (int r = first + 1; r <= last; ++r)
         if (cost(r) < 0.95 * cost(best)) best = r;
@@ -962,7 +969,7 @@ extern "C" int batteries_mace_forward(const float* positions, const float* box,
         row_ptr, N, C, reinterpret_cast<float4*>(out));
     if (N_edges == 0) return (int)hipGetLastError();
     MaceShape sh;
-    int rc = mace_shape(mace_fused_forward_kernel, kMaceFwdWaves, C, &sh);
+    int rc = mace_shape(mace_fused_forward_kernel, kMaceFwdWaves, C, N_edges, &sh);
     if (rc != BM_OK) return rc;
     rc = mace_prepare(positions, mace_box(box), w1, b1, src, dst, row_ptr, order, N, N_edges,
                       cutoff, sh, w, false, stream);
@@ -992,7 +999,7 @@ extern "C" int batteries_mace_backward(const float* positions, const float* box,
         return (int)hipGetLastError();
     }
     MaceShape sh;
-    int rc = mace_shape(mace_fused_backward_kernel, kMaceBwdWaves, C, &sh);
+    int rc = mace_shape(mace_fused_backward_kernel, kMaceBwdWaves, C, N_edges, &sh);
     if (rc != BM_OK) return rc;
     rc = mace_prepare(positions, mace_box(box), w1, b1, src, dst, row_ptr, order, N, N_edges,
                       cutoff, sh, w, true, stream);

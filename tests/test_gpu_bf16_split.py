@@ -25,10 +25,11 @@ def _layer(dev, n, c, seed, scale=1.0):
     return pos, cell, graph, layer, x, go
 
 
-# C: one quad and part of it, 20 quads (three ranges per XCD), 33 quads (more than one
-# round); scale: weights whose lower parts reach down to 2^-100 and up to 2^100
-@pytest.mark.parametrize("n,c,scale", [(60, 1, 1.0), (60, 7, 1.0), (150, 80, 1.0), (40, 130, 1.0),
-                                       (60, 8, 2.0 ** -80), (60, 8, 2.0 ** 100)])
+# C: one quad and part of it, 20 quads (one range per XCD for few edges, three for many), 33
+# quads (more than one round); scale: weights whose lower parts reach down to 2^-100 and up to
+# 2^100
+@pytest.mark.parametrize("n,c,scale", [(60, 1, 1.0), (60, 7, 1.0), (150, 80, 1.0), (400, 80, 1.0),
+                                       (40, 130, 1.0), (60, 8, 2.0 ** -80), (60, 8, 2.0 ** 100)])
 def test_layer_error_against_float64(bm, dev, n, c, scale):
     pos, cell, graph, layer, x, go = _layer(dev, n, c, 31, scale)
     p = pos.to(dev).requires_grad_(True)
