@@ -8,6 +8,9 @@
 // and two rotations of 66 (Passaro and Zitnick, "Reducing SO(3) convolutions to SO(2) for
 // efficient equivariant GNNs", ICML 2023).
 //
+// The rotations mix the components of a degree: an infinite weight of l3 > 0, or an infinite
+// component of x, comes out NaN in every component of its degree.
+//
 // D = (tilt about x) (turn about y): with u = (s sin f, c, s cos f) the turn by f mixes
 // components m and -m, the tilt by the angle of (c, s) the components m >= 0 and those
 // m < 0 among themselves (kTilt).

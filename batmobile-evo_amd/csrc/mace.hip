@@ -643,7 +643,7 @@ __global__ void mace_worker_starts_kernel(const int64_t* __restrict__ pos0, int6
 // h = silu(B(r) W1 + b1); with sg, also s[k] = silu'(z_k) sum_b W1[b][k] dB_b/dr.
 // Sixteen lanes per position: lane q evaluates Bessel function q % 8 (one sincos)
 // and shares it with the position's other lanes, then forms hidden units
-// 4q .. 4q + 3, so every store instruction writes whole 256-byte rows.
+// 4q .. 4q + 3, so every store instruction writes whole 128-byte rows.
 constexpr int kPrepPositions = 16;  // positions per 256-thread workgroup
 __global__ __launch_bounds__(256) void mace_prep_kernel(
     const float* __restrict__ pos, MaceBox bx, const int64_t* __restrict__ src,

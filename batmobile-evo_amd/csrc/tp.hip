@@ -225,9 +225,9 @@ __global__ __launch_bounds__(kTpBlock) void tp_simple_backward_kernel(
 //   gy[n,b]     = sum_{ci,q,a} c * x[n,ci,a] * h[n,ci,q]
 //   gW[p,ci,co] = sum_n sum_{q in p} T[n,ci,q] * g[n,co,out(q)]
 //
-// The three channel contractions (out, h, gW) are GEMMs per slot.  Calls with few rows or
-// no workspace run on v_mfma_f32_16x16x4f32 over 16-row tiles as follows; the others take the
-// mixing kernel further below.  The CG contractions (T, gx, gy) run
+// The three channel contractions (out, h, gW) are GEMMs per slot.  gW, and out and h in calls
+// with few rows or no workspace, run on v_mfma_f32_16x16x4f32 over 16-row tiles as follows; the
+// others take the mixing kernel further below (mix_forward_rows, mix_backward_rows).  The CG contractions (T, gx, gy) run
 // on the VALU with compile-time coefficients.  Each kernel splits the slots
 // into groups taken by different workgroups, so that a group's
 // outputs are disjoint from the others':
@@ -755,7 +755,8 @@ __global__ __launch_bounds__(512) void tp_weighted_bwd_xy_mfma_kernel(
 // on the bf16 matrix cores (common.h), after which the CG entries of p are applied on the
 // VALU: out[o] += c y[b] h_p[a], or gx[a] += c y[b] h_p[o] and gy[b] += c x[a] h_p[o].
 // Mixing before the CG contraction keeps Z, 16 values a row and channel, the operand that
-// is split and staged; contracted first, it is 156.
+// is split and staged; contracted first, it is 156.  (An infinite weight of a path whose Z
+// side has l > 0 makes h infinite with both signs, and their sum over the components NaN.)
 //
 // Workgroup: 16 rows, 8 waves.  Up to 64 contracted channels of Z sit in LDS as operand
 // fragments sZ[(z * KS + s) * 3 + part][lane] (row lane % 16, channels 32 s + 8 (lane / 16)

@@ -15,8 +15,9 @@ is the per-edge-weight form of the same pattern:
 computed by the HIP kernels of the library: one fused kernel per pass that forms
 each tile of per-edge weights R on MFMA (h W2) and consumes it in the channel-wise
 CG product and the scatter-add without storing it (R would take 34 C floats per
-edge, 26 GB at configs[4]); the backward runs the transpose GEMM of the MLP on
-MFMA in the same tiles and ends in per-edge position gradients.
+edge, 26 GB at configs[4]); the backward forms R and its derivative along the edge's
+length the same way and ends in per-edge position gradients.  Lengths are bounded
+below by 1e-10 (u = v / 1e-10 for shorter edges, the length then a constant).
 Gradients are provided for the positions only (forces); the layer's weights
 and the node features are treated as constants.
 """

@@ -40,6 +40,7 @@ SETTLE_STEPS = 500     # untimed launches before the warmup (GPU clock ramp)
 METRIC = "fused SH+TP+scatter edges/s (N=5k,C=64,~30 nbr) + % of HBM/MFMA roofline"
 HBM_PEAK_GBS = 8000.0
 MFMA_FP32_PEAK_TFLOPS = 157.3
+MFMA_BF16_PEAK_TFLOPS = 16 * MFMA_FP32_PEAK_TFLOPS
 N_ATOMS, CHANNELS, CUTOFF = 5000, 64, 5.0
 RHO = 30.0 / (4.0 / 3.0 * math.pi * CUTOFF ** 3)
 SEED = 3
@@ -192,7 +193,11 @@ def other_configs(torch, bm, dev):
     f = 20000 * (624 * 32 * 64 + 3666 * 32)
     res["cfg2_tp_weighted_bwd_ms"] = round(t, 5)
     res["cfg2_tp_weighted_bwd_TFLOPs"] = round(f / (t * 1e-3) / 1e12, 2)
-    res["cfg2_tp_weighted_bwd_mfma_frac"] = round(f / (t * 1e-3) / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4)
+    # grad_W and the CG terms at the fp32 rate, grad_x / grad_y's channel mixing as six bf16
+    # products each
+    mix = 20000 * 312 * 32 * 64
+    res["cfg2_tp_weighted_bwd_mfma_frac"] = round(
+        ((f - mix) / MFMA_FP32_PEAK_TFLOPS + 6 * mix / MFMA_BF16_PEAK_TFLOPS) / (t * 1e-3) / 1e12, 4)
     return res
 
 
@@ -298,8 +303,9 @@ def mace_config4(torch, bm, dev, reps=3):
     graph, forward, backward w.r.t. positions (one fused kernel per pass; the per-edge
     weights R = h W2 are formed on MFMA per tile and never stored).  Flop model per edge:
     radial MLP 2 (8 64 + 64 34 C) and channel-wise CG product (1222 + 312) C forward; the
-    backward recomputes R and runs the MLP's transpose GEMM (twice the MLP) and twice the
-    CG work."""
+    backward forms R again and its derivative along the length (twice the MLP) and twice the
+    CG work.  The matrix cores' share counts the six bf16 products that each fp32 product of
+    those GEMMs takes."""
     n, c = 50000, 128
     g = torch.Generator().manual_seed(4)
     L = (n / RHO) ** (1.0 / 3.0)
@@ -338,16 +344,16 @@ def mace_config4(torch, bm, dev, reps=3):
     mlp = 2 * (8 * 64 + 64 * 34 * c)
     f_fwd = e * (mlp + (1222 + 312) * c)
     f_bwd = e * (2 * mlp + 2 * (1222 + 312) * c)
-    mfma_fwd = e * 2 * 64 * 34 * c          # R = h W2 on MFMA
-    mfma_bwd = 2 * mfma_fwd                 # R again, and g_h = gR W2^T
+    mfma_fwd = 6 * e * 2 * 64 * 34 * c      # R = h W2
+    mfma_bwd = 2 * mfma_fwd                 # R again, and S = s W2
     return {
         "cfg4_mace_N": n, "cfg4_mace_C": c, "cfg4_mace_E": e,
         "cfg4_mace_graph_build_ms": round(build, 3),
         "cfg4_mace_fwd_ms": round(t_f * 1e3, 3), "cfg4_mace_bwd_ms": round(t_b * 1e3, 3),
         "cfg4_mace_fwd_TFLOPs": round(f_fwd / t_f / 1e12, 2),
         "cfg4_mace_bwd_TFLOPs": round(f_bwd / t_b / 1e12, 2),
-        "cfg4_mace_fwd_mfma_part_frac": round(mfma_fwd / t_f / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4),
-        "cfg4_mace_bwd_mfma_part_frac": round(mfma_bwd / t_b / 1e12 / MFMA_FP32_PEAK_TFLOPS, 4),
+        "cfg4_mace_fwd_mfma_part_frac": round(mfma_fwd / t_f / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4),
+        "cfg4_mace_bwd_mfma_part_frac": round(mfma_bwd / t_b / 1e12 / MFMA_BF16_PEAK_TFLOPS, 4),
         "cfg4_mace_peak_device_GB": round(peak / 1e9, 2),
     }
 

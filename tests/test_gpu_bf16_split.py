@@ -46,8 +46,9 @@ def test_layer_error_against_float64(bm, dev, n, c, scale):
 
 
 def test_infinite_weight_stays_infinite(bm, dev):
-    """An infinite W2 entry makes the same outputs infinite (not NaN) as the fp32 product
-    R = h W2 does: path 0 (l1 = l2 = l_out = 0) of channel 1, hidden unit 5."""
+    """An infinite W2 entry of path 0 (l1 = l2 = l_out = 0, which no rotation mixes with other
+    components) makes the same outputs infinite (not NaN) as the fp32 product R = h W2 does:
+    channel 1, hidden unit 5."""
     pos, cell, graph, layer, x, _ = _layer(dev, 80, 4, 41)
     layer.W2[5, 0 * 4 + 1] = float("inf")
     out = layer(graph, pos.to(dev), x.to(dev)).cpu()
