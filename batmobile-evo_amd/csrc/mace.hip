@@ -639,6 +639,15 @@ __global__ void mace_worker_starts_kernel(const int64_t* __restrict__ pos0, int6
     wstart[w] = min(pos0[lo], n_edges);
 }
 
+// (a, b), of unit length but for rounding, closer to it: the rotations take up to the sixth
+// power of what its length is off.
+__device__ __forceinline__ void unit2(float& a, float& b) {
+    const float big = fmaxf(fabsf(a), fabsf(b)), small = fminf(fabsf(a), fabsf(b));
+    const float e = 0.5f * fmaf(-small, small, fmaf(-big, big, 1.0f));
+    a = fmaf(a, e, a);
+    b = fmaf(b, e, b);
+}
+
 // Per position p (edge e = perm[p]): direction (and length), source, destination,
 // h = silu(B(r) W1 + b1); with sg, also s[k] = silu'(z_k) sum_b W1[b][k] dB_b/dr.
 // Sixteen lanes per position: lane q evaluates Bessel function q % 8 (one sincos)
@@ -670,7 +679,7 @@ __global__ __launch_bounds__(256) void mace_prep_kernel(
         // The off-axis part is scaled before it is squared: below 1e-19 its square is
         // subnormal, and (cos f, sin f) would not be of unit length.
         const float m = fmaxf(fabsf(v[0]), fabsf(v[2]));
-        float cf = 1.0f, sf = 0.0f, s2 = fabsf(v[0] + v[2]);  // (0, or NaN)
+        float cf = 1.0f, sf = 0.0f, c = v[1], s2 = fabsf(v[0] + v[2]);  // (0, or NaN)
         if (m > 0.0f) {
             sf = v[0] / m;
             cf = v[2] / m;
@@ -679,11 +688,13 @@ __global__ __launch_bounds__(256) void mace_prep_kernel(
             cf *= ih;
             s2 = m * h;
         }
-        float c = v[1];
         if (r <= kMinLength) {  // (marked: mace_frame; also a NaN, which stays one)
             if (s2 < 1e-15f && fabsf(c) < 1e-15f) c = s2 = 0.0f;  // (its square is subnormal)
             s2 = copysignf(s2, -1.0f);
+        } else {
+            unit2(c, s2);
         }
+        unit2(cf, sf);
         u4[p] = make_float4(cf, sf, c, s2);
         srcp[p] = (int)s;
         dstp[p] = (int)d;
